@@ -663,6 +663,36 @@ int prep_conv_flat(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const vo
   return prep_dense(ctx, cs, x, w, scale, shift, cout, ho, wo, a, out);
 }
 
+// A layout conversion (pack.hip) of n images of h x w pixels and c channels
+// between the NCHW float32 tensor at `flat` and NHWC rows of `pitch` elements
+// at `rows`.  The 8-channel tile (512 pixels) serves tensors of up to 8
+// channels (images); a 64-channel tile of 64 pixels would leave 7/8 of its
+// lanes without a channel there.
+static int prep_layout(vrs_ctx* ctx, const char* op, int dtype, vrs_pack_args& a, int n, int c, int h, int w,
+                       int pitch, const void* flat, const void* rows, std::vector<Launch>& out) {
+  int rc;
+  const int64_t hw = (int64_t)h * w;
+  const bool pack = !strcmp(op, "pack");
+  const int cols = pack ? pitch : c;   // channels written (pack: the zero padding too) or read
+  const int ct = cols <= 8 ? 8 : 64, pt = 4096 / ct;
+  a.N = n; a.C = c; a.HW = hw; a.c_pad = pitch;
+  const int64_t tp = (hw + pt - 1) / pt;
+  a.tiles_c = (cols + ct - 1) / ct;
+  const int epc = 16 / elt_size(dtype);
+  a.vec_p = hw % 4 == 0 && reinterpret_cast<uintptr_t>(flat) % 16 == 0;
+  a.vec_c = pitch % epc == 0 && reinterpret_cast<uintptr_t>(rows) % 16 == 0;
+  const int64_t blocks = (int64_t)n * tp * a.tiles_c;
+  if (blocks >= (1ll << 24)) return fail(VRS_EBADSHAPE, "%s: grid too large", op);   // 2^32 threads
+  a.tiles_p = (int32_t)tp;
+  char name[48];
+  snprintf(name, sizeof name, "vrs_%s_nchw_%s_c%d", op, dsuffix(dtype), ct);
+  hipFunction_t f;
+  if ((rc = get_fn(ctx, name, &f))) return rc;
+  out.push_back(make_launch(name, f, dim3((unsigned)blocks), dim3(256), 0, a));
+  out.back().bytes = (double)n * (double)hw * (4.0 * c + (double)cols * elt_size(dtype));
+  return VRS_OK;
+}
+
 int prep_pack_input(vrs_ctx* ctx, const float* x, int n, int c, int h, int w, const vrs_nhwc& y, int dtype,
                     std::vector<Launch>& out) {
   int rc;
@@ -672,15 +702,10 @@ int prep_pack_input(vrs_ctx* ctx, const float* x, int n, int c, int h, int w, co
   if (y.n != n || y.h != h || y.w != w || y.c < c || y.c >= c + 8)
     return fail(VRS_EBADSHAPE, "pack_input: output view %dx%dx%dx%d for input %dx%dx%dx%d (c padded by < 8)", y.n,
                 y.h, y.w, y.c, n, c, h, w);
-  vrs_pack_args a{x, y.data, n, c, h, w, y.c};
-  char name[48];
-  snprintf(name, sizeof name, "vrs_pack_nchw_%s", dsuffix(dtype));
-  hipFunction_t f;
-  if ((rc = get_fn(ctx, name, &f))) return rc;
-  const int64_t threads = (int64_t)n * h * w;
-  out.push_back(make_launch(name, f, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, a));
-  out.back().bytes = (double)n * h * w * (4.0 * c + (double)y.c * elt_size(dtype));
-  return VRS_OK;
+  vrs_pack_args a{};
+  a.x = x;
+  a.y = y.data;
+  return prep_layout(ctx, "pack", dtype, a, n, c, h, w, y.c, x, y.data, out);
 }
 
 int prep_unpack(vrs_ctx* ctx, const vrs_nhwc& x, int dtype, float* y, std::vector<Launch>& out) {
@@ -689,17 +714,9 @@ int prep_unpack(vrs_ctx* ctx, const vrs_nhwc& x, int dtype, float* y, std::vecto
   if ((rc = check_view(x, "unpack input", 1))) return rc;
   if (!y) return fail(VRS_EINVAL, "unpack: null output");
   vrs_pack_args a{};
-  a.x = static_cast<const float*>(at(x, dtype));
+  a.x = at(x, dtype);
   a.y = y;
-  a.N = x.n; a.C = x.c; a.H = x.h; a.W = x.w; a.c_pad = x.pitch;
-  char name[48];
-  snprintf(name, sizeof name, "vrs_unpack_nchw_%s", dsuffix(dtype));
-  hipFunction_t f;
-  if ((rc = get_fn(ctx, name, &f))) return rc;
-  const int64_t threads = (int64_t)x.n * x.c * x.h * x.w;
-  out.push_back(make_launch(name, f, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, a));
-  out.back().bytes = (double)threads * (4.0 + elt_size(dtype));
-  return VRS_OK;
+  return prep_layout(ctx, "unpack", dtype, a, x.n, x.c, x.h, x.w, x.pitch, y, a.x, out);
 }
 
 int prep_pool(vrs_ctx* ctx, const vrs_nhwc& buf, int dtype, std::vector<Launch>& out) {
@@ -1003,7 +1020,7 @@ int prep_pwpair(vrs_ctx* ctx, const vrs_nhwc& x, const void* w1, const float* s1
   a.w2 = w2; a.s2 = s2; a.b2 = b2;
   a.y = y;
   a.y_sb = sb; a.y_sp = sp; a.y_sc = sc;
-  a.M = (int32_t)M; a.HW = (int32_t)hw; a.NC = nc;
+  a.M = (int32_t)M; a.HW = hw; a.NC = nc;
   a.x_pitch = x.pitch; a.x_bytes = (int32_t)xb; a.y_bytes = (int32_t)(last * 4);
   // maps of at least two tiles per CU: the weight-stationary persistent
   // kernel (one 8-wave group per CU, W1 and W2 in registers); smaller ones:

@@ -166,11 +166,16 @@ typedef struct {
 } vrs_up_args;
 
 /* NCHW float32 image batch -> NHWC element-type buffer with c_pad channels
- * (channels >= C are zero). */
+ * (channels >= C are zero), or back (unpack: x the NHWC view's first channel,
+ * y float32 NCHW, C the view's channels, c_pad the source's pitch). */
 typedef struct {
-  const float* x;
+  const void* x;
   void* y;
-  int32_t N, C, H, W, c_pad;
+  int64_t HW;     /* pixels per image */
+  int32_t N, C, c_pad;
+  int32_t tiles_p, tiles_c; /* pixel and channel tiles per image */
+  int32_t vec_p;  /* float32 side: 16-byte accesses of 4 pixels (HW % 4 == 0, aligned base) */
+  int32_t vec_c;  /* NHWC side: 16-byte accesses of whole channel chunks (aligned base and pitch) */
 } vrs_pack_args;
 
 /* PSA attention, key_dim 32, head_dim 64 (blocks/c2psa.rs:61-116).

@@ -295,42 +295,6 @@ VRS_CONV_KERNEL(vrs_conv_f32_32x256_k32_a, float, 32, 256, 32, 1, 4, true)
 VRS_CONV_KERNEL(vrs_conv_f32_32x256_k32_g, float, 32, 256, 32, 1, 4, false)
 
 // ---------------------------------------------------------------------------
-// NCHW float32 image batch -> NHWC (element type) with zero channel padding.
-// One thread per output pixel; the c_pad (<= 8) channels go out as one group.
-template <typename T>
-__device__ __forceinline__ void pack_body(const vrs_pack_args& a) {
-  const int64_t HW = (int64_t)a.H * a.W;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)a.N * HW) return;
-  const int64_t b = i / HW, p = i - b * HW;
-  T* y = reinterpret_cast<T*>(a.y) + i * a.c_pad;
-  for (int c = 0; c < a.c_pad; ++c) {
-    const float v = c < a.C ? a.x[(b * a.C + c) * HW + p] : 0.f;
-    y[c] = Elt<T>::from_f(v);
-  }
-}
-
-extern "C" __global__ __launch_bounds__(256) void vrs_pack_nchw_bf16(vrs_pack_args a) { pack_body<bf16_t>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_pack_nchw_f32(vrs_pack_args a) { pack_body<float>(a); }
-
-// NHWC view (element type) -> NCHW float32, one thread per output element.
-template <typename T>
-__device__ __forceinline__ void unpack_body(const vrs_pack_args& a) {
-  // reuse of vrs_pack_args: x = source view base (pre-offset), y = float32 NCHW,
-  // N, C (channels of the view), H, W, c_pad = source pitch
-  const int64_t HW = (int64_t)a.H * a.W;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)a.N * a.C * HW) return;
-  const int64_t p = i % HW, bc = i / HW;
-  const int64_t c = bc % a.C, b = bc / a.C;
-  const T* src = reinterpret_cast<const T*>(a.x);
-  reinterpret_cast<float*>(a.y)[i] = Elt<T>::to_f(src[(b * HW + p) * a.c_pad + c]);
-}
-
-extern "C" __global__ __launch_bounds__(256) void vrs_unpack_nchw_bf16(vrs_pack_args a) { unpack_body<bf16_t>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_unpack_nchw_f32(vrs_pack_args a) { unpack_body<float>(a); }
-
-// ---------------------------------------------------------------------------
 // Stem (model.0 = conv(3, c, 3, 2), yolo26/mod.rs:126-195) fused with the
 // input layout change: 3x3 stride-2 pad-1 conv straight from the NCHW float32
 // image, folded BN + activation, NHWC output of the element type.
