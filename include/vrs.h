@@ -128,6 +128,16 @@ typedef struct {
  * vrs_conv_pointwise_pair launch; the first conv then has no launch and no
  * output of its own. */
 #define VRS_TILE_PWPAIR 13
+/* Split-K kernels for small problems (bf16 and float32, k up to 5, any
+ * stride, fused upsample and flat outputs included): one 32x32 or 16x16 output
+ * tile per workgroup, whose waves share the K range and sum their parts in a
+ * fixed order.  OR one of VRS_TILE_SPLIT(n) for the number of waves sharing K:
+ * 1 (16x16 only: four neighbouring tiles per workgroup), 4 or 8; none: by the
+ * depth of K. */
+#define VRS_TILE_KW32 14
+#define VRS_TILE_KW16 15
+#define VRS_TILE_SPLIT(n) ((n) == 1 ? 0x1000 : (n) == 4 ? 0x2000 : 0x3000)
+#define VRS_TILE_SPLIT_MASK 0xf000
 #define VRS_TILE_K32 0x100
 /* OR VRS_TILE_PERSIST: persistent grid (resident workgroups loop over the
  * tiles with one continuous load stream, so a tile's epilogue overlaps the

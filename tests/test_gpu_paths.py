@@ -41,3 +41,81 @@ def test_layout_conversions_exact(dtype, n, c, c_pad, h, w, shift):
         ctx().unpack_output(vrs.nhwc(y, c - off, off), dtype, back[shift:].view(n, c - off, h, w))
         torch.cuda.synchronize()
         assert np.array_equal(back[shift:].cpu().numpy().reshape(n, c - off, h, w), rounder(dtype)(x)[:, off:])
+
+
+SPLIT_TILES = [pytest.param(vrs.TILE_KW16 | vrs.TILE_SPLIT_1, id="16x4"),
+               pytest.param(vrs.TILE_KW16 | vrs.TILE_SPLIT_4, id="16w4"),
+               pytest.param(vrs.TILE_KW16 | vrs.TILE_SPLIT_8, id="16w8"),
+               pytest.param(vrs.TILE_KW32 | vrs.TILE_SPLIT_4, id="32w4"),
+               pytest.param(vrs.TILE_KW32 | vrs.TILE_SPLIT_8, id="32w8")]
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("tile", SPLIT_TILES)
+@pytest.mark.parametrize("case", [
+    # n, cin, h, w, cout, k, s, residual
+    (1, 8, 1, 1, 4, 1, 1, False),       # one pixel, one chunk of K: most waves have no step
+    (1, 8, 5, 3, 20, 3, 1, True),       # 15 pixels, 20 channels; taps of one chunk
+    (2, 24, 4, 4, 36, 3, 2, False),     # taps that do not fill a step, 8 pixels
+    (1, 32, 8, 8, 32, 3, 1, True),      # whole 32x32 tiles; float32: one step per tap
+    (1, 64, 3, 11, 33 * 4, 3, 1, False),  # 33 pixels, bfloat16: one step per tap
+    (3, 72, 6, 7, 64, 1, 1, True),      # 126 pixels: the last of four neighbouring tiles is partial
+    (1, 128, 7, 9, 48, 5, 1, False),    # 25 taps
+    (1, 512, 4, 5, 16, 3, 2, False),    # deep K: several rounds of steps per wave
+])
+def test_split_k_conv(case, tile, dtype):
+    import zlib
+
+    import oracle
+    import torch
+    from gpu_util import dev, from_nhwc, rel_err, to_nhwc
+    n, cin, h, w, cout, k, s, with_res = case
+    rnd = rounder(dtype)
+    rng = np.random.default_rng(zlib.crc32(repr(case).encode()))
+    x = rnd(rng.standard_normal((n, cin, h, w)).astype(np.float32))
+    wt = rnd((rng.standard_normal((cout, cin, k, k)) * np.sqrt(2.0 / (cin * k * k))).astype(np.float32))
+    scale = rng.uniform(0.5, 1.5, cout).astype(np.float32)
+    shift = rng.normal(0, 0.2, cout).astype(np.float32)
+    ho, wo = (h - 1) // s + 1, (w - 1) // s + 1
+    ref = oracle.affine_act(oracle.conv2d(x, wt, s, k // 2), scale, shift, 1)
+    res = rnd(rng.standard_normal(ref.shape).astype(np.float32)) if with_res else None
+    xt = to_nhwc(x, dtype, cin + 8, 8)
+    yt = torch.full((n, ho, wo, cout + 8), 7.0, dtype=tdtype(dtype), device="cuda")
+    rt = to_nhwc(res, dtype, cout + 4, 4) if with_res else None
+    ctx().conv2d(vrs.nhwc(xt, cin, 8), dev(vrs.pack_conv_weight(wt, 1, cin, dtype)), dev(scale), dev(shift),
+                 vrs.nhwc(yt, cout, 4), k, s, 1, vrs.ACT_SILU, vrs.nhwc(rt, cout, 4) if with_res else None, dtype,
+                 tile=tile)
+    torch.cuda.synchronize()
+    # the bounds of the other conv kernels (float32: eps * sqrt(K) products in another order)
+    err = rel_err(from_nhwc(yt, cout, 4), ref + res if with_res else ref, 5e-2 if dtype == vrs.F32 else 1e-1)
+    assert err < (1e-4 if dtype == vrs.F32 else 2e-2), err
+    assert torch.all(yt[..., :4] == 7.0) and torch.all(yt[..., cout + 4:] == 7.0)
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("tile", SPLIT_TILES)
+def test_split_k_network(tile, dtype):
+    """Every dense conv of YOLO26n on a split-K tile (fused upsamples and the
+    Detect head's flat outputs included) against the 128x128 tile."""
+    import torch
+    from vrs.synth import images, seeded_params
+    desc = vrs.block(vrs.BLOCK_YOLO26, 3, nc=7, variant="n")
+    x = torch.from_numpy(images(2, 64, 96)).cuda()
+    outs = []
+    for code in (vrs.TILE_128x128, tile):
+        m = vrs.Model(ctx(), desc, 2, 64, 96, dtype, 1e-3, autotune=False)
+        P = seeded_params(m.params(), seed=3, bn="random")
+        stem = {i for i, (p, _, _) in enumerate(m.conv_info()) if p == "model.0"}
+        w = {p[: -len(".conv.weight")] if p.endswith(".conv.weight") else p[: -len(".weight")]: v.shape
+             for p, v in P.items() if v.ndim == 4}
+        m.set_plan([0 if i in stem or w[p][1] == 1 else code for i, (p, _, _) in enumerate(m.conv_info())])
+        m.load(P)
+        outs.append([o.double().cpu() for o in m.forward(x)])
+        names = m.launch_names()
+    kernel = "_s32_w" if tile & 0xff == vrs.TILE_KW32 else "_s16_w"
+    assert sum(kernel in s for s in names) > 70, names
+    for a, b in zip(*outs):
+        # float32: ~100 layers of another summation order, 1e-6 each; bfloat16:
+        # roundings that flip and travel on, 0.5 % of a deep network's outputs
+        rel = float((a - b).norm() / a.norm())
+        assert rel < (1e-4 if dtype == vrs.F32 else 2e-2), rel

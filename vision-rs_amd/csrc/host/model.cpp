@@ -1089,9 +1089,9 @@ int autotune_tiles(vrs_model* m) {
     const Buf& xb = m->bufs[c.x.buf];
     const int64_t npix = (int64_t)m->batch * ((xb.h + 2 * (c.k / 2) - c.k) / c.s + 1) *
                          ((xb.w + 2 * (c.k / 2) - c.k) / c.s + 1);
-    const std::vector<int> cand =
+    std::vector<int> cand =
         conv_tile_candidates(c.cout, c.cin, dt, c.k, c.s, c.has_up ? 0 : xb.w, npix, m->ctx->num_cu);
-    if (cand.size() < 2) continue;
+    if (cand.empty()) continue;
     if (c.out_idx >= 0 && !outs[c.out_idx]) {
       size_t n = 1;
       for (int32_t d : m->out_dims[c.out_idx]) n *= (size_t)d;
@@ -1105,6 +1105,16 @@ int autotune_tiles(vrs_model* m) {
     cs.k = c.k; cs.stride = c.s; cs.dtype = dt; cs.act = c.kind == CK_BN_SILU ? VRS_ACT_SILU : VRS_ACT_NONE;
     cs.in_scale = 1.f;  // timing only: values do not matter
     if (pass) e4m3_flags(m, c, cs);   // the storage planned for the forced fp8 model
+    // A small conv's tile is the automatic one when that is a split-K tile,
+    // without a contest: these sum K in another order than the other tiles,
+    // and float32 results must not depend on a timing (all other float32
+    // tiles give the same bits).
+    {
+      std::vector<Launch> ls;
+      if (prep_conv_step(m, c, cs, pass ? c.w8 : c.w, pass ? c.scale8 : c.scale, outs.data(), ls) == VRS_OK &&
+          split_k_tile(ls[0].tile))
+        cand = {ls[0].tile};
+    }
     float best = 1e30f;
     int best_tile = VRS_TILE_AUTO;
     for (int t : cand) {

@@ -96,14 +96,15 @@ static int resident_wgs(hipFunction_t f, int threads = 256) {
 }
 
 // Dense-conv tiles.  bf16 has every tile with 32- and (when Cin % 64 == 0)
-// 64-deep K steps; the float32 parity path has 128x128, 64x256 and 32x256.
+// 64-deep K steps; the float32 parity path has 128x128, 64x256, 64x64 and
+// 32x256.
 struct TileInfo { int code, bm, bn; const char* tag; bool f32; bool k32; int threads; };
 static const TileInfo kTiles[] = {
     {VRS_TILE_128x128, 128, 128, "128x128", true, true, 256}, {VRS_TILE_256x128, 256, 128, "256x128", false, true, 256},
     {VRS_TILE_128x256, 128, 256, "128x256", false, true, 256}, {VRS_TILE_64x256, 64, 256, "64x256", true, true, 256},
     {VRS_TILE_32x256, 32, 256, "32x256", true, true, 256},
     {VRS_TILE_256x256, 256, 256, "256x256", false, false, 512},  // 64-deep K steps only
-    {VRS_TILE_64x64, 64, 64, "64x64", false, true, 256},          // bf16, Cin % 32 == 0
+    {VRS_TILE_64x64, 64, 64, "64x64", true, true, 256},           // Cin % 32 == 0
 };
 
 static const TileInfo* tile_info(int code) {
@@ -113,9 +114,9 @@ static const TileInfo* tile_info(int code) {
 }
 
 // Kernel name for a tile, or an error when the combination is not built.
-// up: the fused-upsample instance (_u), built for 128x128, 256x128, 128x256
-// and 256x256 in bf16 and 128x128 and 64x256 in float32, aligned and not
-// persistent
+// up: the fused-upsample instance (_u), built for 128x128, 256x128, 128x256,
+// 256x256 and (64-deep steps) 64x64 in bf16 and 128x128, 64x256 and 64x64 in
+// float32, aligned and not persistent
 static int tile_kernel(int code, int cin, int dtype, bool up, char* name, size_t n, int* bm, int* bn, int* threads,
                        bool x8 = false, bool y8 = false) {
   if ((code & 0xff) == VRS_TILE_H3 || (code & 0xff) == VRS_TILE_W1_256 || (code & 0xff) == VRS_TILE_W1_128)
@@ -124,8 +125,10 @@ static int tile_kernel(int code, int cin, int dtype, bool up, char* name, size_t
   if (!t) return fail(VRS_EINVAL, "conv: unknown tile code %d", code);
   if (up) {
     const bool built = dtype != VRS_F32 ? (t->code == VRS_TILE_128x128 || t->code == VRS_TILE_256x128 ||
-                                           t->code == VRS_TILE_128x256 || t->code == VRS_TILE_256x256)
-                                        : (t->code == VRS_TILE_128x128 || t->code == VRS_TILE_64x256);
+                                           t->code == VRS_TILE_128x256 || t->code == VRS_TILE_256x256 ||
+                                           (t->code == VRS_TILE_64x64 && !(code & VRS_TILE_K32)))
+                                        : (t->code == VRS_TILE_128x128 || t->code == VRS_TILE_64x256 ||
+                                           t->code == VRS_TILE_64x64);
     if (!built || (code & VRS_TILE_PERSIST) || cin % 32 != 0)
       return fail(VRS_EUNSUPPORTED, "conv: no fused-upsample kernel for tile %s (dtype %d, Cin %d)", t->tag, dtype, cin);
   }
@@ -171,20 +174,6 @@ static int tile_kernel(int code, int cin, int dtype, bool up, char* name, size_t
   return VRS_OK;
 }
 
-// Shape heuristic (VRS_TILE_AUTO): the widest tile that still gives the
-// 256-CU chip at least two workgroups per CU.
-static int auto_tile(int cout, int cin, int64_t M, int dtype, int num_cu) {
-  auto blocks = [&](int bm, int bn) { return (int64_t)((cout + bm - 1) / bm) * ((M + bn - 1) / bn); };
-  const int64_t want = 2ll * (num_cu > 0 ? num_cu : 256);
-  if (cout <= 32) return VRS_TILE_32x256;
-  if (cout <= 64) return VRS_TILE_64x256;
-  if (dtype == VRS_BF16 && cin % 32 == 0) {
-    if (cout <= 128 && blocks(128, 256) >= want) return VRS_TILE_128x256;
-    if (cout > 128 && blocks(256, 128) >= want) return VRS_TILE_256x128;
-  }
-  return VRS_TILE_128x128;
-}
-
 // Strip width of the halo-tiled 3x3 kernel for an image width (0: not usable).
 // 32 or 16 when they divide the width: a 16-lane group of the MFMA operand
 // reads then never spans a strip row (a row change skips the two halo
@@ -199,6 +188,159 @@ static int h3_strip_width(int w) {
   if (w <= 40) return w;
   if (w % 20 == 0) return 20;
   return 32;
+}
+
+// Predicted time of one conv on one tile (microseconds at 256 CUs), for the
+// automatic choice and to prune the autotuner's candidates:
+//   c0 + c1 * nk + c2 * wk * g + c3 * g + c4 * MB / 4,
+// nk the K steps (of 32 elements, or 128 bytes on the split-K tiles) in a
+// row, wk those of one workgroup over all its waves, g the workgroups per CU,
+// MB the operands' bytes: the launch, the chain of dependent steps, the
+// throughput once several workgroups share a CU, the epilogue, HBM.  Fitted to
+// 250 measured shapes (batch 1..64, 10..160 pixels a side, 16..1024 channels,
+// 1x1 and 3x3) on every tile of both types; median error 4-10 %.  Steps: '6'
+// 64-deep, '3' 32-deep, 'g' Cin not in whole steps, 'a' in whole steps.  The
+// tile it picks is 2 % over the best one (geometric mean), where the rule it
+// replaces (the widest tile that leaves two workgroups per CU) was 1.64x over
+// it in bfloat16 and 2.7x in float32.
+struct TileCost { int dtype, tile; char steps; float c[5]; };
+static const TileCost kTileCost[] = {
+    {VRS_BF16, VRS_TILE_128x128, 'g', {4.18, 0.543, 0.193, 1.62, 0.188}},
+    {VRS_BF16, VRS_TILE_128x128, '3', {4.48, 0.248, 0.172, 1.97, 0}},
+    {VRS_BF16, VRS_TILE_128x128, '6', {4.67, 0.205, 0.143, 2.39, 0}},
+    {VRS_BF16, VRS_TILE_128x256, '3', {6.39, 0.382, 0.444, 2.91, 0.00949}},
+    {VRS_BF16, VRS_TILE_128x256, '6', {6.5, 0.519, 0.298, 6, 0}},
+    {VRS_BF16, VRS_TILE_256x128, '3', {6.2, 0.357, 0.4, 2.48, 0.132}},
+    {VRS_BF16, VRS_TILE_256x128, '6', {6.39, 0.318, 0.201, 6.48, 0.0455}},
+    {VRS_BF16, VRS_TILE_256x256, '6', {8.83, 0.5, 0.177, 7.29, 0.246}},
+    {VRS_BF16, VRS_TILE_32x256, 'g', {3.71, 0.607, 0.246, 1.08, 0}},
+    {VRS_BF16, VRS_TILE_32x256, '3', {3.5, 0.439, 0.191, 1.18, 0}},
+    {VRS_BF16, VRS_TILE_64x256, 'g', {4.38, 0.67, 0.279, 1.78, 0.0421}},
+    {VRS_BF16, VRS_TILE_64x256, '3', {4.9, 0.308, 0.29, 1.2, 0.154}},
+    {VRS_BF16, VRS_TILE_64x256, '6', {4.97, 0.275, 0.217, 4.56, 0}},
+    {VRS_BF16, VRS_TILE_64x64, '3', {3.14, 0.159, 0.0942, 0.552, 0}},
+    {VRS_BF16, VRS_TILE_64x64, '6', {3.17, 0.116, 0.0726, 0.718, 0}},
+    {VRS_BF16, VRS_TILE_H3, 0, {5.79, 0.152, 0.0886, 3.06, 0}},
+    {VRS_BF16, VRS_TILE_KW16 | VRS_TILE_SPLIT(1), 'a', {2.89, 0.159, 0.125, 0.505, 0.102}},
+    {VRS_BF16, VRS_TILE_KW16 | VRS_TILE_SPLIT(1), 'g', {2.89, 0.202, 0.133, 0.516, 0.0638}},
+    {VRS_BF16, VRS_TILE_KW16 | VRS_TILE_SPLIT(4), 'a', {3.07, 0.194, 0.0296, 0.497, 0.00987}},
+    {VRS_BF16, VRS_TILE_KW16 | VRS_TILE_SPLIT(4), 'g', {2.92, 0.221, 0.0367, 0.461, 0}},
+    {VRS_BF16, VRS_TILE_KW16 | VRS_TILE_SPLIT(8), 'a', {3.06, 0.25, 0.0311, 1.18, 0}},
+    {VRS_BF16, VRS_TILE_KW16 | VRS_TILE_SPLIT(8), 'g', {2.88, 0.276, 0.034, 1.1, 0}},
+    {VRS_BF16, VRS_TILE_KW32 | VRS_TILE_SPLIT(4), 'a', {3.79, 0.293, 0.0667, 1.13, 0}},
+    {VRS_BF16, VRS_TILE_KW32 | VRS_TILE_SPLIT(4), 'g', {3.46, 0.389, 0.0795, 1.07, 0}},
+    {VRS_BF16, VRS_TILE_KW32 | VRS_TILE_SPLIT(8), 'a', {3.49, 0.36, 0.0866, 3.06, 0}},
+    {VRS_BF16, VRS_TILE_KW32 | VRS_TILE_SPLIT(8), 'g', {3.15, 0.54, 0.0928, 2.98, 0}},
+    {VRS_BF16, VRS_TILE_W1_128, 0, {3.02, 0.287, 0.0197, 1.15, 0.248}},
+    {VRS_BF16, VRS_TILE_W1_256, 0, {4.37, 0.335, 0, 1.06, 0.656}},
+    {VRS_F32, VRS_TILE_128x128, 'g', {3.9, 2.09, 1.54, 6.2, 0}},
+    {VRS_F32, VRS_TILE_128x128, '3', {5.63, 1.85, 1.03, 4.79, 0.246}},
+    {VRS_F32, VRS_TILE_32x256, 'g', {2.01, 1.53, 1.46, 4.64, 0}},
+    {VRS_F32, VRS_TILE_32x256, '3', {3.91, 1.25, 0.875, 5.31, 0}},
+    {VRS_F32, VRS_TILE_64x256, 'g', {4.43, 2.4, 1.77, 10.7, 0}},
+    {VRS_F32, VRS_TILE_64x256, '3', {5.29, 2.04, 1.04, 8.79, 0}},
+    {VRS_F32, VRS_TILE_64x64, '3', {3.13, 0.493, 0.398, 1.66, 0}},
+    {VRS_F32, VRS_TILE_KW16 | VRS_TILE_SPLIT(1), 'a', {3.03, 0.249, 0.159, 0.682, 0.102}},
+    {VRS_F32, VRS_TILE_KW16 | VRS_TILE_SPLIT(1), 'g', {2.41, 0.25, 0.197, 0.722, 0.161}},
+    {VRS_F32, VRS_TILE_KW16 | VRS_TILE_SPLIT(4), 'a', {3.22, 0.248, 0.0439, 0.551, 0}},
+    {VRS_F32, VRS_TILE_KW16 | VRS_TILE_SPLIT(4), 'g', {3.1, 0.236, 0.0484, 0.569, 0}},
+    {VRS_F32, VRS_TILE_KW16 | VRS_TILE_SPLIT(8), 'a', {3.15, 0.327, 0.0461, 1.26, 0}},
+    {VRS_F32, VRS_TILE_KW16 | VRS_TILE_SPLIT(8), 'g', {3.28, 0.298, 0.0473, 1.32, 0}},
+    {VRS_F32, VRS_TILE_KW32 | VRS_TILE_SPLIT(4), 'a', {4.27, 0.484, 0.143, 1.29, 0}},
+    {VRS_F32, VRS_TILE_KW32 | VRS_TILE_SPLIT(4), 'g', {3.47, 0.392, 0.146, 1.4, 0}},
+    {VRS_F32, VRS_TILE_KW32 | VRS_TILE_SPLIT(8), 'a', {4.13, 0.578, 0.158, 3.22, 0}},
+    {VRS_F32, VRS_TILE_KW32 | VRS_TILE_SPLIT(8), 'g', {3.16, 0.384, 0.163, 3.57, 0}},
+};
+
+struct ConvShape { int cout, cin, k, dtype; int64_t m, in_px; };
+
+static double tile_cost(const ConvShape& s, int tile, int64_t h3_blocks, int num_cu) {
+  const int code = tile & 0xff, es = (int)elt_size(s.dtype);
+  const bool kw = code == VRS_TILE_KW32 || code == VRS_TILE_KW16;
+  const bool k64 = s.dtype == VRS_BF16 && s.cin % 64 == 0 && !(tile & VRS_TILE_K32) && code != VRS_TILE_32x256;
+  char steps = kw ? (s.cin * es % 128 == 0 ? 'a' : 'g') : s.cin % 32 ? 'g' : k64 ? '6' : '3';
+  int bm, bn;
+  if (code == VRS_TILE_H3) bm = s.cout <= 32 ? 32 : 64, bn = 256, steps = 0;
+  else if (code == VRS_TILE_W1_256 || code == VRS_TILE_W1_128) bm = code == VRS_TILE_W1_256 ? 256 : 128, bn = 64, steps = 0;
+  else if (code == VRS_TILE_KW32) bm = bn = 32;
+  else if (code == VRS_TILE_KW16) bm = 16, bn = (tile & VRS_TILE_SPLIT_MASK) == VRS_TILE_SPLIT(1) ? 64 : 16;
+  else if (const TileInfo* t = tile_info(code)) bm = t->bm, bn = t->bn;
+  else return 1e30;
+  const int key = kw ? tile : code;
+  for (const TileCost& t : kTileCost) {
+    if (t.dtype != s.dtype || t.tile != key || t.steps != steps) continue;
+    const int K = s.k * s.k * s.cin;
+    double nk, wk;
+    if (kw) {
+      const int split = (tile & VRS_TILE_SPLIT_MASK) == VRS_TILE_SPLIT(1)   ? 1
+                        : (tile & VRS_TILE_SPLIT_MASK) == VRS_TILE_SPLIT(4) ? 4
+                                                                            : 8;
+      wk = (K * es + 127) / 128;
+      nk = ((int)wk + split - 1) / split;
+    } else {
+      const int bk = k64 ? 64 : 32;
+      nk = wk = (double)((K + bk - 1) / bk) * (bk / 32);
+    }
+    const double blocks = code == VRS_TILE_H3 && h3_blocks > 0
+                              ? (double)h3_blocks
+                              : (double)((s.cout + bm - 1) / bm) * (double)((s.m + bn - 1) / bn);
+    const double g = blocks / (num_cu > 0 ? num_cu : 256);
+    const double mb = ((double)s.in_px * s.cin + (double)s.m * s.cout + (double)s.cout * K) * es * 1e-6;
+    return t.c[0] + t.c[1] * nk + t.c[2] * wk * g + t.c[3] * g + t.c[4] * mb / 4;
+  }
+  return 1e30;
+}
+
+static const int kSplitTiles[] = {VRS_TILE_KW16 | VRS_TILE_SPLIT(1), VRS_TILE_KW16 | VRS_TILE_SPLIT(4),
+                                  VRS_TILE_KW16 | VRS_TILE_SPLIT(8), VRS_TILE_KW32 | VRS_TILE_SPLIT(4),
+                                  VRS_TILE_KW32 | VRS_TILE_SPLIT(8)};
+
+// VRS_TILE_AUTO: the tile of the least predicted time among those built for
+// the conv; the widest tile that gives the chip two workgroups per CU stays
+// unless another is predicted 10 % faster (the model's error).
+// staged: the output is an NHWC view the staged stores take (a.stage == 1).
+static int auto_tile(const ConvSpec& cs, const vrs_conv_args& a, const vrs_nhwc& x, int num_cu) {
+  const ConvShape s{a.Cout, a.Cin, a.kh, cs.dtype, a.M, (int64_t)x.n * x.h * x.w};
+  const bool staged = a.stage == 1 && !a.y_f32, g = a.Cin % 32 != 0;
+  const int64_t want = 2ll * (num_cu > 0 ? num_cu : 256);
+  auto blocks = [&](int bm, int bn) { return (int64_t)((s.cout + bm - 1) / bm) * ((s.m + bn - 1) / bn); };
+  int best = VRS_TILE_128x128;
+  if (!cs.up) {
+    if (s.cout <= 32) best = VRS_TILE_32x256;
+    else if (s.cout <= 64) best = VRS_TILE_64x256;
+    else if (s.dtype == VRS_BF16 && !g && s.cout <= 128 && blocks(128, 256) >= want) best = VRS_TILE_128x256;
+    else if (s.dtype == VRS_BF16 && !g && s.cout > 128 && blocks(256, 128) >= want) best = VRS_TILE_256x128;
+  }
+  double t = 0.9 * tile_cost(s, best, 0, num_cu);
+  auto offer = [&](int tile, int64_t h3_blocks = 0) {
+    const double u = tile_cost(s, tile, h3_blocks, num_cu);
+    if (u < t) t = u, best = tile;
+  };
+  for (const TileInfo& ti : kTiles) {
+    if (s.dtype == VRS_F32 && !ti.f32) continue;
+    if (g && ti.code != VRS_TILE_128x128 && ti.code != VRS_TILE_64x256 && ti.code != VRS_TILE_32x256) continue;
+    if (!ti.k32 && a.Cin % 64) continue;
+    if (cs.up && ti.code != VRS_TILE_128x128 && (ti.code != VRS_TILE_64x64 || (s.dtype == VRS_BF16 && a.Cin % 64)))
+      continue;
+    offer(ti.code);
+  }
+  const int cps = 128 / (int)elt_size(s.dtype);
+  if (a.kh <= 5 && (!cs.up || (a.Cin % cps == 0 && a.c_split % cps == 0)))
+    for (int tile : kSplitTiles) offer(tile);
+  const int tw = h3_strip_width(x.w);
+  if (s.dtype == VRS_BF16 && a.kh == 3 && a.stride == 1 && !g && tw && !cs.up && staged && a.res_bytes >= 0 &&
+      (int64_t)x.n * x.h * x.w * (int64_t)x.pitch * 2 < (1ll << 31)) {
+    // (strips that pad the map by more than a fifth are left out: the runs'
+    // padding costs more there than the fitted shapes show)
+    const int64_t runs = (int64_t)((x.w + tw - 1) / tw) * (((int64_t)x.h * tw + 255) / 256);
+    if (5 * runs * 256 <= 6ll * x.h * x.w)
+      offer(VRS_TILE_H3, runs * x.n * ((s.cout + (s.cout <= 32 ? 31 : 63)) / (s.cout <= 32 ? 32 : 64)));
+  }
+  if (s.dtype == VRS_BF16 && a.kh == 1 && a.stride == 1 && !cs.up && a.Cin % 64 == 0 && !a.res && staged) {
+    if (a.Cin <= 192) offer(VRS_TILE_W1_256);
+    if (a.Cin <= 256 || a.Cin == 384) offer(VRS_TILE_W1_128);
+  }
+  return best;
 }
 
 // Input widths the fp8 weight-stationary 1x1 kernel is built for.
@@ -231,7 +373,7 @@ std::vector<int> conv_tile_candidates(int cout, int cin, int dtype, int k, int s
     if (dtype == VRS_F32 && !t.f32) continue;
     if (g && t.code != VRS_TILE_128x128 && t.code != VRS_TILE_64x256 && t.code != VRS_TILE_32x256) continue;
     if (t.bm >= 2 * 128 && cout <= 128) continue;   // mostly empty rows
-    if (t.bm <= 64 && cout > 4 * t.bm) continue;     // too many passes over the input
+    if (t.bm <= 64 && t.bn > 64 && cout > 4 * t.bm) continue;   // too many passes over the input
     if (t.code == VRS_TILE_64x64) {   // only where 128x128 leaves the chip under-filled
       const int64_t b128 = (int64_t)((cout + 127) / 128) * ((m + 127) / 128);
       if (g || (m > 0 && b128 >= 2ll * (num_cu > 0 ? num_cu : 256))) continue;
@@ -250,12 +392,75 @@ std::vector<int> conv_tile_candidates(int cout, int cin, int dtype, int k, int s
       if (t.code == VRS_TILE_128x128 && cin % 64 == 0) c.push_back(t.code | VRS_TILE_PERSIST);
     }
   }
+  // leave out the tiles predicted to take over 1.4 times the best one's time
+  // (nine predictions in ten are within 27 % of the measured time): finalize
+  // times a third to a half of the built tiles
+  if (m > 0) {
+    const ConvShape s{cout, cin, k, dtype, m, m * stride * stride};
+    double best = 1e30;
+    for (int t : c) best = std::min(best, tile_cost(s, t & ~VRS_TILE_PERSIST, 0, num_cu));
+    c.erase(std::remove_if(c.begin(), c.end(),
+                           [&](int t) { return tile_cost(s, t & ~VRS_TILE_PERSIST, 0, num_cu) > 1.4 * best; }),
+            c.end());
+  }
   return c;
 }
 
-static int prep_dense(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w, const float* scale,
+// Split-K small-problem kernel (convk.hip) on prep_dense's argument block.
+static int prep_splitk(vrs_ctx* ctx, const ConvSpec& cs, int cout, vrs_conv_args& a, std::vector<Launch>& out) {
+  const int ts = (cs.tile & 0xff) == VRS_TILE_KW32 ? 32 : 16;
+  if (cs.dtype != VRS_BF16 && cs.dtype != VRS_F32)
+    return fail(VRS_EUNSUPPORTED, "conv: the split-K tiles take bf16 or float32 (dtype %d)", cs.dtype);
+  if (cs.tile & ~(0xff | VRS_TILE_SPLIT_MASK))
+    return fail(VRS_EINVAL, "conv: tile code %d: the split-K tiles take only VRS_TILE_SPLIT flags", cs.tile);
+  if (cs.k > 5) return fail(VRS_EUNSUPPORTED, "conv: the split-K tiles take k <= 5 (k=%d)", cs.k);
+  const int es = (int)elt_size(cs.dtype), cps = 128 / es;   // channels per 128-byte step
+  vrs_convk_args k{};
+  k.gpt = a.Cin * es / 16;
+  const bool aligned = a.Cin % cps == 0;
+  if (a.c_split && (!aligned || a.c_split % cps))
+    return fail(VRS_EUNSUPPORTED, "conv: split-K tile with a fused upsample needs Cin and the split in %d channels", cps);
+  const int steps = (a.K * es + 127) / 128;
+  int kw = 0;
+  switch (cs.tile & VRS_TILE_SPLIT_MASK) {
+    case 0: kw = steps >= 24 ? 8 : steps >= 4 || ts == 32 ? 4 : 1; break;
+    case VRS_TILE_SPLIT(1): kw = 1; break;
+    case VRS_TILE_SPLIT(4): kw = 4; break;
+    case VRS_TILE_SPLIT(8): kw = 8; break;
+    default: return fail(VRS_EINVAL, "conv: unknown K split in tile code %d", cs.tile);
+  }
+  if (kw == 1 && ts == 32) return fail(VRS_EUNSUPPORTED, "conv: the 32x32 split-K tile shares K over 4 or 8 waves");
+  const int nt = kw == 1 ? 4 : 1;
+  a.tiles_m = (cout + ts - 1) / ts;
+  a.tiles_n = (a.M + ts * nt - 1) / (ts * nt);
+  k.c = a;
+  k.d_chunk = 8 * kw % k.gpt;
+  k.d_tap = 8 * kw / k.gpt;
+  k.inv_kw = (256 + cs.k - 1) / cs.k;
+  // the operand with more bytes is read by as few XCDs as the order allows
+  k.chan_major = a.w_bytes > (int64_t)a.N * a.H * a.W * a.Cin * es;
+  const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
+  if (blocks >= (1ll << 31) / 1024) return fail(VRS_EBADSHAPE, "conv: grid too large for the split-K tile");
+  char name[48];
+  snprintf(name, sizeof name, "vrs_conv_%s_s%d_w%d_%c", dsuffix(cs.dtype), ts, kw, aligned ? 'a' : 'g');
+  hipFunction_t f;
+  if (int rc = get_fn(ctx, name, &f)) return rc;
+  out.push_back(make_launch(name, f, dim3((unsigned)blocks), dim3(64 * kw * nt), 0, k));
+  const double cin = cs.cin_real > 0 ? cs.cin_real : a.Cin, kk = (double)cs.k * cs.k;
+  const double cin_up = cs.up ? (double)cs.up->c : 0.0;   // read at a quarter of the pixels
+  out.back().flops = 2.0 * (double)a.M * cout * kk * cin;
+  out.back().bytes = (double)a.N * a.H * a.W * (cin - 0.75 * cin_up) * es + (double)cout * kk * cin * es +
+                     (double)a.M * cout * (a.y_f32 ? 4.0 : es) + (a.res ? (double)a.M * cout * es : 0.0) + 8.0 * cout;
+  return VRS_OK;
+}
+
+static int prep_tile(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, int cout, vrs_conv_args& a,
+                     std::vector<Launch>& out);
+
+static int prep_dense(vrs_ctx* ctx, const ConvSpec& spec, const vrs_nhwc& x, const void* w, const float* scale,
                       const float* shift, int cout, int ho, int wo, vrs_conv_args& a, std::vector<Launch>& out) {
   int rc;
+  ConvSpec cs = spec;
   const bool f8 = cs.dtype == VRS_FP8;
   if (!f8 && (rc = check_dtype(cs.dtype))) return rc;
   if (!f8 && (cs.x_f8 || cs.y_f8 || cs.res_f8))
@@ -325,6 +530,21 @@ static int prep_dense(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const
     return fail(VRS_EBADSHAPE, "conv: %lld output pixels per launch exceed 2^24 (split the batch)", (long long)M);
   a.M = (int32_t)M;
   a.act = cs.act;
+  if (!cs.tile)
+    cs.tile = f8 ? (cout <= 64 && !cs.up ? VRS_TILE_64x256 : VRS_TILE_128x128) : auto_tile(cs, a, x, ctx->num_cu);
+  const size_t first = out.size();
+  if ((rc = prep_tile(ctx, cs, x, cout, a, out))) return rc;
+  for (size_t i = first; i < out.size(); ++i) out[i].tile = cs.tile;
+  return VRS_OK;
+}
+
+// The launches of one dense conv on tile cs.tile (not VRS_TILE_AUTO), from
+// prep_dense's checked argument block.
+static int prep_tile(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, int cout, vrs_conv_args& a,
+                     std::vector<Launch>& out) {
+  int rc;
+  const bool f8 = cs.dtype == VRS_FP8;
+  const int64_t xs = cs.x_f8 ? 1 : (int64_t)elt_size(cs.dtype), M = a.M;
   char name[64];
   int bm, bn, threads;
   if ((cs.tile & 0xff) == VRS_TILE_H3) {
@@ -409,10 +629,9 @@ static int prep_dense(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const
                        8.0 * cout;
     return VRS_OK;
   }
-  const int tile = cs.tile ? cs.tile
-                            : f8 ? (cout <= 64 && !cs.up ? VRS_TILE_64x256 : VRS_TILE_128x128)
-                                 : cs.up ? VRS_TILE_128x128   // built in every fused-upsample dtype
-                                         : auto_tile(cout, x.c, M, cs.dtype, ctx->num_cu);
+  if (split_k_tile(cs.tile))
+    return prep_splitk(ctx, cs, cout, a, out);
+  const int tile = cs.tile;
   if ((rc = tile_kernel(tile, x.c, cs.dtype, cs.up != nullptr, name, sizeof name, &bm, &bn, &threads, cs.x_f8,
                         cs.y_f8)))
     return rc;

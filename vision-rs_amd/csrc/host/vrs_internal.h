@@ -71,6 +71,7 @@ struct Launch {
   std::vector<uint8_t> args;
   double flops = 0.0;  // algorithmic work of this launch
   double bytes = 0.0;  // compulsory HBM bytes (inputs + weights + outputs)
+  int tile = VRS_TILE_AUTO;  // dense convs: the tile in use (VRS_TILE_AUTO resolved)
 };
 
 int run(const Launch& l, hipStream_t s);
@@ -140,7 +141,9 @@ int prep_absmax(vrs_ctx* ctx, const vrs_nhwc& x, unsigned* out, std::vector<Laun
 uint8_t f32_to_e4m3(float v);
 // Dense conv tiles worth trying for a layer (autotuning candidates).
 // m: output pixels (0: unknown), num_cu: the device's CUs
+// The split-K tiles (VRS_TILE_KW*) are not among them: see split_k_tile.
 std::vector<int> conv_tile_candidates(int cout, int cin, int dtype, int k, int stride, int w, int64_t m, int num_cu);
+inline bool split_k_tile(int tile) { return (tile & 0xff) == VRS_TILE_KW32 || (tile & 0xff) == VRS_TILE_KW16; }
 int prep_conv(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w, const float* scale,
               const float* shift, const vrs_nhwc* res, const vrs_nhwc& y, std::vector<Launch>& out);
 // Dense conv storing float32 into a strided (flat) output: element (b, p, co)

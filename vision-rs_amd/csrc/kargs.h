@@ -76,6 +76,16 @@ typedef struct {
   int32_t res_f8;
 } vrs_conv_args;
 
+/* Split-K small-problem conv (convk.hip): tiles_m x tiles_n output tiles; a
+ * filter tap's Cin channels are gpt 16-byte chunks; a wave's next step is
+ * d_tap taps and d_chunk chunks on (with a carry of at most one tap). */
+typedef struct {
+  vrs_conv_args c;
+  int32_t gpt, d_chunk, d_tap;
+  int32_t inv_kw;     /* ceil(256 / kw): tap / kw == tap * inv_kw >> 8 for kw 1, 3, 5 and tap < kw * kw */
+  int32_t chan_major; /* workgroup order: pixel tiles of one channel tile together */
+} vrs_convk_args;
+
 /* Fused bottleneck pair (bf16): y = act2(s2 * conv3x3(w2, act1(s1 * conv3x3(w1,
  * x) + b1)) + b2) + res, both convs 3x3 stride 1 pad 1 with SiLU, the middle
  * map never leaving the workgroup.  x, y, res: NHWC views of N x H x W pixels

@@ -271,6 +271,8 @@ VRS_CONV_KERNEL_U(vrs_conv_bf16_256x128_k64_u, bf16_t, 256, 128, 64, 2, 2)
 VRS_CONV_KERNEL_U(vrs_conv_bf16_128x256_k32_u, bf16_t, 128, 256, 32, 2, 2)
 VRS_CONV_KERNEL_U(vrs_conv_bf16_128x256_k64_u, bf16_t, 128, 256, 64, 2, 2)
 VRS_CONV_KERNEL_U(vrs_conv_bf16_256x256_k64_u, bf16_t, 256, 256, 64, 2, 4)
+VRS_CONV_KERNEL_U(vrs_conv_bf16_64x64_k64_u, bf16_t, 64, 64, 64, 2, 2)
+VRS_CONV_KERNEL_U(vrs_conv_f32_64x64_k32_u, float, 64, 64, 32, 2, 2)
 VRS_CONV_KERNEL_U(vrs_conv_f32_128x128_k32_u, float, 128, 128, 32, 2, 2)
 VRS_CONV_KERNEL_U(vrs_conv_f32_64x256_k32_u, float, 64, 256, 32, 1, 4)
 #define VRS_CONV_P(NAME, BM, BN, BK, WGM, WGN)                                                   \
@@ -289,6 +291,7 @@ extern "C" __global__ __launch_bounds__(512, 2) void vrs_conv_bf16_256x256_k64_p
 // f32 (parity path, fp32 MFMA)
 VRS_CONV_KERNEL(vrs_conv_f32_128x128_k32_a, float, 128, 128, 32, 2, 2, true)
 VRS_CONV_KERNEL(vrs_conv_f32_128x128_k32_g, float, 128, 128, 32, 2, 2, false)
+VRS_CONV_KERNEL(vrs_conv_f32_64x64_k32_a, float, 64, 64, 32, 2, 2, true)
 VRS_CONV_KERNEL(vrs_conv_f32_64x256_k32_a, float, 64, 256, 32, 1, 4, true)
 VRS_CONV_KERNEL(vrs_conv_f32_64x256_k32_g, float, 64, 256, 32, 1, 4, false)
 VRS_CONV_KERNEL(vrs_conv_f32_32x256_k32_a, float, 32, 256, 32, 1, 4, true)
