@@ -119,3 +119,31 @@ def test_split_k_network(tile, dtype):
         # roundings that flip and travel on, 0.5 % of a deep network's outputs
         rel = float((a - b).norm() / a.norm())
         assert rel < (1e-4 if dtype == vrs.F32 else 2e-2), rel
+
+
+@pytest.mark.parametrize("dtype,n,c,h,w,s", [
+    # LDS tile: strips of 4 rows, 64 bytes of channels, tiles of 4..40 x 10..40
+    (vrs.F32, 1, 8, 1, 1, 1), (vrs.F32, 1, 24, 45, 50, 1), (vrs.F32, 2, 40, 21, 41, 2), (vrs.F32, 30, 96, 33, 37, 1),
+    (vrs.BF16, 1, 8, 2, 9, 1), (vrs.BF16, 1, 40, 45, 50, 1), (vrs.BF16, 9, 136, 21, 23, 1),
+    # row walker (more than 40 MB moved): 10-row bands, and 40-row bands with a 1-row last one
+    (vrs.BF16, 12, 320, 33, 90, 1), (vrs.BF16, 16, 264, 41, 75, 1),
+])
+def test_depthwise_paths(dtype, n, c, h, w, s):
+    import oracle
+    import torch
+    from gpu_util import dev, from_nhwc, rel_err, to_nhwc
+    rnd = rounder(dtype)
+    rng = np.random.default_rng([n, c, h, w, s])
+    x = rnd(rng.standard_normal((n, c, h, w), dtype=np.float32))
+    wt = rnd((rng.standard_normal((c, 1, 3, 3)) * 0.4).astype(np.float32))
+    scale = rng.uniform(0.5, 1.5, c).astype(np.float32)
+    shift = rng.normal(0, 0.2, c).astype(np.float32)
+    ref = oracle.affine_act(oracle.conv2d(x, wt, s, 1, c), scale, shift, 1)
+    xt = to_nhwc(x, dtype, c + 8, 8)
+    yt = torch.full((n, ref.shape[2], ref.shape[3], c + 8), 7.0, dtype=tdtype(dtype), device="cuda")
+    ctx().conv2d(vrs.nhwc(xt, c, 8), dev(vrs.pack_conv_weight(wt, c, 1, dtype)), dev(scale), dev(shift),
+                 vrs.nhwc(yt, c, 0), 3, s, c, vrs.ACT_SILU, None, dtype)
+    torch.cuda.synchronize()
+    err = rel_err(from_nhwc(yt, c, 0), ref, 5e-2 if dtype == vrs.F32 else 1e-1)   # bounds of the other depthwise tests
+    assert err < (1e-4 if dtype == vrs.F32 else 2e-2), err
+    assert torch.all(yt[..., c:] == 7.0)

@@ -778,6 +778,45 @@ static int prep_grouped(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, con
   return VRS_OK;
 }
 
+// Output tile of the LDS-tile depthwise kernel (tile_h x tile_w and the tile
+// counts of `a`); returns the workgroups.  Least predicted time: the latency
+// of one workgroup (t[0] + t[1] per round of 512 input pixels + t[2] per round
+// of 64 strips) plus, for each further workgroup per CU, its share of loads
+// (t[3]), strips (t[4]) and start (t[5]); microseconds, fitted to 17 shapes x
+// up to 30 tiles per kernel (rms error 8-10 %; the tile it picks is 2-4 % over
+// the best).
+static int64_t dw_tile(int dtype, int stride, int n, int c, int ho, int wo, int num_cu, vrs_dw_args& a) {
+  static const double kBf16[6] = {2.57, 1.11, 1.92, 0.894, 0.638, 1.19}, kF32[6] = {2.26, 1.10, 1.90, 1.76, 0.294, 0.421},
+                      kF32s2[6] = {3.01, 1.32, 0.893, 1.14, 0.037, 0.477};
+  const double* t = dtype == VRS_BF16 ? kBf16 : stride == 1 ? kF32 : kF32s2;
+  // (float32 stride 1: three workgroups share a CU's LDS up to 44 KB)
+  const int cap = dtype == VRS_F32 && stride == 1 ? 44 * 1024 : 64 * 1024;
+  const int64_t blocks = ((int64_t)c * (int64_t)elt_size(dtype) + 63) / 64;
+  double best = 1e30;
+  int64_t wgs = 0;
+  for (int th0 : {4, 8, 12, 16, 20, 40})
+    for (int tw0 : {10, 16, 20, 32, 40}) {
+      const int th = std::min(th0, ho), tw = std::min(tw0, wo);
+      const int px = ((th - 1) * stride + 3) * ((tw - 1) * stride + 3);
+      if (px * 64 > cap) continue;
+      const int64_t wg = n * blocks * ((ho + th - 1) / th) * ((wo + tw - 1) / tw);
+      const double strips = ((th + 3) / 4 * tw + 63) / 64;
+      const double us = t[0] + t[1] * ((px + 511) / 512) + t[2] * strips +
+                        std::max(0.0, (double)wg / (num_cu > 0 ? num_cu : 256) - 1.0) *
+                            (t[3] * px / 512 + t[4] * strips + t[5]);
+      if (us < best) {
+        best = us;
+        wgs = wg;
+        a.tile_h = th;
+        a.tile_w = tw;
+        a.cblocks = (int32_t)blocks;
+        a.bands = (ho + th - 1) / th;
+        a.patches = (wo + tw - 1) / tw;
+      }
+    }
+  return wgs;
+}
+
 int prep_conv(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w, const float* scale,
               const float* shift, const vrs_nhwc* res, const vrs_nhwc& y, std::vector<Launch>& out) {
   int rc;
@@ -803,26 +842,38 @@ int prep_conv(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w
     char name[48];
     hipFunction_t f;
     const int64_t xb = ((int64_t)x.n * x.h * x.w * x.pitch - x.c_off) * (int64_t)elt_size(cs.dtype);
-    if (cs.stride == 1 && xb < (1ll << 31)) {
-      // row-walking kernel: bands of 40 output rows on maps of 32 rows or
-      // more (few band halos and per-wave start-ups: 80 and 40 rows divide
-      // evenly), 10 on small ones (enough waves to fill the chip)
-      const int rb = x.h >= 32 ? 40 : 10;
+    const int64_t moved = ((int64_t)x.n * x.h * x.w + (int64_t)y.n * y.h * y.w) * x.c * (int64_t)elt_size(cs.dtype);
+    a.cblocks = (x.c + 63) / 64;
+    a.patches = (x.w + 7) / 8;
+    // waves of the row walker on 40-row bands
+    const int64_t walk40 = (int64_t)x.n * ((x.h + 39) / 40) * a.cblocks * a.patches;
+    const int64_t per_img = (int64_t)((y.h + 3) / 4) * y.w * (x.c / 8);   // 4-row strips of 8 channels
+    if (cs.stride == 2 && per_img >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: map too large for one grid row");
+    if (cs.dtype == VRS_BF16 && cs.stride == 2) {
+      if ((rc = get_fn(ctx, "vrs_dwconv3_s2_bf16", &f))) return rc;
+      out.push_back(make_launch("vrs_dwconv3_s2_bf16", f, dim3((unsigned)((per_img + 255) / 256), (unsigned)x.n),
+                                dim3(256), 0, a));
+    } else if (cs.dtype == VRS_BF16 && cs.stride == 1 && xb < (1ll << 31) && moved > (40ll << 20)) {
+      // Row-walking kernel: over 40 MB moved it is as fast as the LDS tile or
+      // faster (45 MB 17.5 vs 20.4 us, 52 MB 19.9 vs 19.9, 210 MB 52 vs 57;
+      // at 26 MB 12.4 vs 11.4).  Bands of 40 output rows on maps of 32 rows or
+      // more when that leaves four waves per CU (few band halos and per-wave
+      // start-ups; 640 waves 25 us, the same in 10-row bands 18-21 us), else 10.
+      const int rb = x.h >= 32 && walk40 >= 4ll * (ctx->num_cu > 0 ? ctx->num_cu : 256) ? 40 : 10;
       a.x_bytes = (int32_t)xb;
-      a.cblocks = (x.c + 63) / 64;
-      a.patches = (x.w + 7) / 8;
       a.bands = (x.h + rb - 1) / rb;
       const int64_t wgs = (int64_t)x.n * a.bands * a.cblocks * ((a.patches + 3) / 4);
-      if (wgs >= (1ll << 31)) return fail(VRS_EBADSHAPE, "dwconv: grid too large");
-      snprintf(name, sizeof name, "vrs_dwconv3_s1w%d_%s", rb, dsuffix(cs.dtype));
+      if (wgs >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: grid too large");
+      snprintf(name, sizeof name, "vrs_dwconv3_s1w%d_bf16", rb);
       if ((rc = get_fn(ctx, name, &f))) return rc;
       out.push_back(make_launch(name, f, dim3((unsigned)wgs), dim3(256), 0, a));
     } else {
-      const int64_t per_img = (int64_t)((y.h + 3) / 4) * y.w * (x.c / 8);
-      if (per_img >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: map too large for one grid row");
-      snprintf(name, sizeof name, "vrs_dwconv3_s%d_%s", cs.stride, dsuffix(cs.dtype));
+      const int64_t wgs = dw_tile(cs.dtype, cs.stride, x.n, x.c, y.h, y.w, ctx->num_cu, a);
+      if (wgs >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: grid too large");
+      const uint32_t lds = (uint32_t)(((a.tile_h - 1) * cs.stride + 3) * ((a.tile_w - 1) * cs.stride + 3) * 64);
+      snprintf(name, sizeof name, "vrs_dwconv3_t%d_%s", cs.stride, dsuffix(cs.dtype));
       if ((rc = get_fn(ctx, name, &f))) return rc;
-      out.push_back(make_launch(name, f, dim3((unsigned)((per_img + 255) / 256), (unsigned)x.n), dim3(256), 0, a));
+      out.push_back(make_launch(name, f, dim3((unsigned)wgs), dim3(256), lds, a));
     }
     const double es = (double)elt_size(cs.dtype);
     out.back().flops = 2.0 * x.n * y.h * y.w * (double)x.c * cs.k * cs.k;

@@ -139,6 +139,9 @@ typedef struct {
   /* row-walking stride-1 kernel: raw-buffer extent of x, 64-channel blocks,
    * 8-column patches and row bands per image */
   int32_t x_bytes, cblocks, patches, bands;
+  /* LDS-tile kernels: output rows and columns of a tile (cblocks 64-byte
+   * channel blocks, patches x bands tiles per image) */
+  int32_t tile_h, tile_w;
 } vrs_dw_args;
 
 /* Grouped conv (1 < groups < channels), NHWC, direct form.  x, y, res point

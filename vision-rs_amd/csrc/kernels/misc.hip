@@ -9,15 +9,18 @@
 // Depthwise 3x3 conv + folded BN (+ SiLU): blocks/conv.rs:75-85 (dwconv) and
 // the PE conv_bn with g = c (blocks/c2psa.rs:66).  Weights are tap-major
 // [9][C] in the element type, so the 9 taps of 8 channels are 9 vector loads.
-// One thread computes 8 channels of DW_ROWS vertically adjacent output pixels;
-// every loop is unrolled at compile time (stride is a template parameter) so
-// weights and accumulators stay in registers, and the (DW_ROWS-1)*S+3 input
-// rows x 3 columns are independent loads in flight together.
+//
+// Stride 2, bfloat16: one thread computes 8 channels of DW_ROWS vertically
+// adjacent output pixels; every loop is unrolled at compile time so weights
+// and accumulators stay in registers, and the (DW_ROWS-1)*S+3 input rows x 3
+// columns are independent loads in flight together.  (Taps of neighbouring
+// outputs share little here, and the LDS tile below was 5-30 % slower.)
 namespace {
 constexpr int DW_ROWS = 4;
 
-template <typename T, int S>
-__device__ __forceinline__ void dw_body(const vrs_dw_args& a) {
+__device__ __forceinline__ void dw2_body(const vrs_dw_args& a) {
+  using T = bf16_t;
+  constexpr int S = 2;
   using E = Elt<T>;
   using G = typename E::group;
   constexpr int NR = (DW_ROWS - 1) * S + 3;
@@ -97,7 +100,7 @@ __device__ __forceinline__ void dw_body(const vrs_dw_args& a) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// Stride-1 depthwise 3x3, row walking.  A wave owns 8 output columns x 64
+// Stride-1 depthwise 3x3, bfloat16, row walking: large problems.  A wave owns 8 output columns x 64
 // channels (lane = channel group g + 8 * column cx) of one band of RB output
 // rows and walks down the band's RB + 2 input rows once: each lane loads its
 // own column (16 bytes per bf16 group), takes the left/right neighbours from
@@ -109,14 +112,13 @@ __device__ __forceinline__ void dw_body(const vrs_dw_args& a) {
 // flight: two waves per SIMD at ~230 registers), and rows past the band are
 // not fetched.  The four waves of a workgroup take adjacent column patches so
 // their edge columns meet in L1.
-template <typename T, int RB>
+template <int RB>
 __device__ __forceinline__ void dww_body(const vrs_dw_args& a) {
+  using T = bf16_t;
   using E = Elt<T>;
   using G = typename E::group;
   constexpr int NW = (int)sizeof(G) / 4;          // dwords per group
-  // prefetch ring slots (rows in flight + 1); float32 rows take twice the
-  // registers, so the parity path keeps three
-  constexpr int NP = sizeof(T) == 2 ? 6 : 3;
+  constexpr int NP = 6;                           // prefetch ring slots (rows in flight + 1)
   static_assert((RB + 2) % NP == 0, "rows per band: RB + 2 must be a multiple of the ring");
   // the accumulator slot of band row u (u % 3) is taken from its prefetch
   // slot u % NP at compile time, which needs NP to be a multiple of 3
@@ -243,15 +245,153 @@ __device__ __forceinline__ void dww_body(const vrs_dw_args& a) {
   }
 }
 
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w40_bf16(vrs_dw_args a) { dww_body<bf16_t, 40>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w10_bf16(vrs_dw_args a) { dww_body<bf16_t, 10>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w40_f32(vrs_dw_args a) { dww_body<float, 40>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w10_f32(vrs_dw_args a) { dww_body<float, 10>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w40_bf16(vrs_dw_args a) { dww_body<40>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w10_bf16(vrs_dw_args a) { dww_body<10>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s2_bf16(vrs_dw_args a) { dw2_body(a); }
 
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1_bf16(vrs_dw_args a) { dw_body<bf16_t, 1>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s2_bf16(vrs_dw_args a) { dw_body<bf16_t, 2>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1_f32(vrs_dw_args a) { dw_body<float, 1>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s2_f32(vrs_dw_args a) { dw_body<float, 2>(a); }
+// ---------------------------------------------------------------------------
+// Depthwise 3x3 through an LDS tile: float32, and bfloat16 stride 1 where the
+// row walker's waves do not fill the chip.  A walker wave takes 12 or 42 rows
+// one after the other, so a small problem took 8 or 23 us whatever its size
+// (float32, with fewer rows in flight, 12 or 39 us).  Here a workgroup takes 64
+// bytes of channels (4 chunks of 16 bytes) of a tile_h x tile_w output tile:
+// all its input chunks are requested at once (eight in flight per thread),
+// written to LDS, and each thread computes strips of DT_R output rows of one
+// column from there, so the time is one memory latency plus the arithmetic.
+// Sums in the walker's order: the same bits.  Measured, walker -> tile:
+// float32 64 channels at 80x80 x 1 38.6 -> 5.2 us, 256 at 80x80 x 32 (419 MB)
+// 117 -> 109 us; stride 2 (one thread per output strip before) 512 at 40x40 x 1
+// 8.5 -> 5.4 us, 256 at 80x80 x 32 77 -> 58 us; bfloat16 64 at 80x80 x 1 22.5 ->
+// 5.2 us, 256 at 80x80 x 4 24.3 -> 12.4 us, 512 at 20x20 x 32 12.5 -> 11.4 us
+// (a copy of it 7.5), 256 at 80x80 x 32 52 -> 57 us (walker kept).
+namespace {
+constexpr int DT_R = 4;   // output rows per thread and strip
+
+template <typename T, int S>
+__device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
+  constexpr int EPC = 16 / (int)sizeof(T);       // channels per chunk
+  constexpr int NR = (DT_R - 1) * S + 3;         // input rows of a strip
+  extern __shared__ __attribute__((aligned(16))) unsigned char dwt_lds[];
+  u32x4_t* tile = reinterpret_cast<u32x4_t*>(dwt_lds);   // [input row][input column][chunk]
+  const int tid = threadIdx.x;
+  int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int cb = wg % a.cblocks; wg /= a.cblocks;
+  const int tx = wg % a.patches; wg /= a.patches;
+  const int ty = wg % a.bands;
+  const int b = wg / a.bands;
+  const int oy0 = ty * a.tile_h, ox0 = tx * a.tile_w;
+  const int ic = (a.tile_w - 1) * S + 3;
+  const int rows = min(a.tile_h, a.Ho - oy0), cols = min(a.tile_w, a.Wo - ox0);
+  const int ir = (rows - 1) * S + 3;
+  const int ch = tid & 3;
+  const int c0 = cb * 4 * EPC + ch * EPC;
+  const bool cok = c0 < a.C;
+
+  // this thread's weights and constants (its chunk is the same for every item)
+  u32x4_t wq[9];
+  const T* wp = reinterpret_cast<const T*>(a.w) + (cok ? c0 : 0);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) wq[k] = *reinterpret_cast<const u32x4_t*>(wp + (int64_t)k * a.C);
+  float sc[EPC], sh[EPC];
+#pragma unroll
+  for (int e = 0; e < EPC; ++e) {
+    sc[e] = a.scale[(cok ? c0 : 0) + e];
+    sh[e] = a.shift[(cok ? c0 : 0) + e];
+  }
+
+  const T* x = reinterpret_cast<const T*>(a.x) + (int64_t)b * a.H * a.W * a.x_pitch + c0;
+  const int iy0 = oy0 * S - 1, ix0 = ox0 * S - 1;
+  const float inv_ic = 1.0f / (float)ic;
+  const int npx = ir * ic;
+  constexpr int NB = 8;
+  for (int p0 = tid >> 2; p0 < npx; p0 += 64 * NB) {
+    u32x4_t v[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int p = p0 + i * 64;
+      int cx;
+      const int ry = fdivmod(min(p, npx - 1), ic, inv_ic, cx);
+      const int iy = iy0 + ry, ix = ix0 + cx;
+      v[i] = (u32x4_t){0, 0, 0, 0};
+      if (p < npx && cok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W)
+        v[i] = *reinterpret_cast<const u32x4_t*>(x + ((int64_t)iy * a.W + ix) * a.x_pitch);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      if (p0 + i * 64 < npx) tile[(p0 + i * 64) * 4 + ch] = v[i];
+  }
+  __syncthreads();
+  if (!cok) return;
+
+  auto chunk = [&](const u32x4_t& q, float (&o)[EPC]) {
+    if constexpr (sizeof(T) == 2) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[2 * e] = __uint_as_float(q[e] << 16);
+        o[2 * e + 1] = __uint_as_float(q[e] & 0xffff0000u);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = __uint_as_float(q[e]);
+    }
+  };
+  float wv[9][EPC];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) chunk(wq[k], wv[k]);
+  T* y = reinterpret_cast<T*>(a.y);
+  const int strips = (rows + DT_R - 1) / DT_R, items = strips * cols;
+  const float inv_cols = 1.0f / (float)cols;
+  for (int it = tid >> 2; it < items; it += 64) {
+    int ox;
+    const int st = fdivmod(it, cols, inv_cols, ox);
+    float acc[DT_R][EPC];
+#pragma unroll
+    for (int r = 0; r < DT_R; ++r)
+#pragma unroll
+      for (int e = 0; e < EPC; ++e) acc[r][e] = 0.f;
+    // (the last strip of a partial tile reads rows past its input: clamped,
+    // and feeding only output rows that are not stored)
+#pragma unroll
+    for (int rr = 0; rr < NR; ++rr) {
+      const int row = min(st * DT_R * S + rr, ir - 1);
+      const u32x4_t* t = tile + (row * ic + ox * S) * 4 + ch;
+#pragma unroll
+      for (int kx = 0; kx < 3; ++kx) {
+        float xv[EPC];
+        chunk(t[kx * 4], xv);
+#pragma unroll
+        for (int r = 0; r < DT_R; ++r) {
+          const int ky = rr - r * S;
+          if (ky < 0 || ky > 2) continue;
+#pragma unroll
+          for (int e = 0; e < EPC; ++e) acc[r][e] += wv[ky * 3 + kx][e] * xv[e];
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < DT_R; ++r) {
+      if (st * DT_R + r >= rows) break;
+      float v[EPC];
+#pragma unroll
+      for (int e = 0; e < EPC; ++e) {
+        v[e] = acc[r][e] * sc[e] + sh[e];
+        if (a.act == VRS_ACT_SILU) v[e] = silu_t<T>(v[e]);
+      }
+      u32x4_t o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = sizeof(T) == 2 ? pack_bf16x2(v[(2 * e) % EPC], v[(2 * e + 1) % EPC]) : __float_as_uint(v[e]);
+      *reinterpret_cast<u32x4_t*>(y + (((int64_t)b * a.Ho + oy0 + st * DT_R + r) * a.Wo + ox0 + ox) * a.y_pitch + c0) = o;
+    }
+  }
+}
+}  // namespace
+
+// (bfloat16: 72 float weights and 8-channel strips take 180 registers; three
+// waves per SIMD spilled, 6.6 against 5.2 us on the smallest problems)
+extern "C" __global__ __launch_bounds__(256, 2) void vrs_dwconv3_t1_bf16(vrs_dw_args a) { dwt_body<bf16_t, 1>(a); }
+extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_t1_f32(vrs_dw_args a) { dwt_body<float, 1>(a); }
+extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_t2_f32(vrs_dw_args a) { dwt_body<float, 2>(a); }
 
 // ---------------------------------------------------------------------------
 // Grouped conv with 1 < groups < channels + folded BN (+ SiLU) (+ residual):
