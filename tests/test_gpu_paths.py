@@ -147,3 +147,32 @@ def test_depthwise_paths(dtype, n, c, h, w, s):
     err = rel_err(from_nhwc(yt, c, 0), ref, 5e-2 if dtype == vrs.F32 else 1e-1)   # bounds of the other depthwise tests
     assert err < (1e-4 if dtype == vrs.F32 else 2e-2), err
     assert torch.all(yt[..., c:] == 7.0)
+
+
+@pytest.mark.parametrize("dtype,b,heads,h,w", [
+    (vrs.F32, 1, 1, 1, 1), (vrs.BF16, 1, 1, 1, 1),          # one key: three of the four waves have none
+    (vrs.F32, 1, 2, 8, 16), (vrs.BF16, 1, 2, 8, 16),        # 128 keys: the last size shared by four waves
+    (vrs.F32, 2, 1, 3, 43), (vrs.BF16, 2, 1, 3, 43),        # 129 keys: eight waves, a chunk of one key
+    (vrs.F32, 1, 1, 23, 23), (vrs.BF16, 1, 1, 23, 23),      # 529 keys: a second round of chunks
+    (vrs.BF16, 16, 4, 24, 24),                              # 2304 workgroups of 16 queries: the streamed kernel
+    (vrs.BF16, 16, 5, 20, 20),                              # 2000: the resident kernel
+])
+def test_attention_paths(dtype, b, heads, h, w):
+    import torch
+    torch.manual_seed(b * 1000 + h * w)
+    c = heads * 64
+    qkv = torch.randn(b, h, w, heads * 128, device="cuda").to(tdtype(dtype))
+    pe_w = (torch.randn(9, c, device="cuda") * 0.3).to(tdtype(dtype))
+    pe_s, pe_t = torch.rand(c, device="cuda") + 0.5, torch.randn(c, device="cuda") * 0.1
+    out = torch.full((b, h, w, c + 8), 7.0, device="cuda", dtype=tdtype(dtype))
+    ctx().psa_attention(vrs.nhwc(qkv), pe_w, pe_s, pe_t, vrs.nhwc(out, c, 4), heads, dtype)
+    q, k, v = qkv.double().reshape(b, h * w, heads, 128).permute(0, 2, 1, 3).split((32, 32, 64), 3)
+    p = (torch.matmul(q.contiguous(), k.transpose(2, 3).contiguous()) * 32 ** -0.5).softmax(-1)
+    o = torch.matmul(p, v.contiguous()).permute(0, 2, 1, 3).reshape(b, h, w, c)
+    vm = torch.nn.functional.pad(v.permute(0, 2, 1, 3).reshape(b, h, w, c), (0, 0, 1, 1, 1, 1))
+    pe = sum(vm[:, i // 3:i // 3 + h, i % 3:i % 3 + w] * pe_w[i].double() for i in range(9))
+    ref = o + pe * pe_s.double() + pe_t.double()
+    # float32: a few roundings of the largest term; bfloat16: the probabilities' and the output's 2^-9
+    err = float((out[..., 4:c + 4].double() - ref).abs().max() / ref.square().mean().sqrt())
+    assert err < (1e-5 if dtype == vrs.F32 else 4e-2), err
+    assert torch.all(out[..., :4] == 7.0) and torch.all(out[..., c + 4:] == 7.0)

@@ -1077,7 +1077,24 @@ int prep_attn(vrs_ctx* ctx, int heads, int dtype, const vrs_nhwc& qkv, const voi
   }
   char name[48];
   int threads;
-  if (dtype == VRS_BF16 && N <= 512 && a.qkv_bytes > 0) {
+  // Split-key kernel (attn.hip): 16 queries per workgroup.  Float32: always
+  // (1.5-4.2x faster than the streamed kernel from 8 to 3200 workgroups, which
+  // stays for images of 2 GiB and more).  bfloat16: while the resident kernel
+  // (up to 512 keys) or the streamed one leaves the chip idle: 20x20 at 4 heads
+  // 800 workgroups 12.6 vs 14.7 us, 1600 20.6 vs 15.3; 37x33 1232 workgroups
+  // 29.7 vs 33.3 us, 30x24 2880 42.8 vs 42.1.  Eight waves share the keys while
+  // that fills at most 8 waves per CU (or there are over 1024 keys), else four:
+  // 20x20 float32 100 workgroups 8.4 vs 8.9 us, 400 14.6 vs 13.6; 9x7 7.0 vs 5.6.
+  const int64_t blocks16 = (int64_t)a.B * heads * ((N + 15) / 16);
+  const int64_t cus = ctx->num_cu > 0 ? ctx->num_cu : 256;
+  const bool image32 = (int64_t)N * qkv.pitch * (int64_t)elt_size(dtype) < (1ll << 31);
+  if (image32 && blocks16 < (1ll << 22) &&
+      (dtype == VRS_F32 || blocks16 <= (N <= 512 && a.qkv_bytes > 0 ? 4 : 8) * cus)) {
+    const int kw = N > 128 && (blocks16 <= cus || (N > 1024 && blocks16 <= 4 * cus)) ? 8 : 4;
+    a.q_blocks = (N + 15) / 16;
+    threads = kw * 64;
+    snprintf(name, sizeof name, "vrs_psa_attn_s%d_%s", kw, dsuffix(dtype));
+  } else if (dtype == VRS_BF16 && N <= 512 && a.qkv_bytes > 0) {
     // the head's K and V^T resident in LDS, one wave per 32 queries: tiles
     // of 7 query tiles (two workgroups per 20x20 head) while those fit in
     // one round over the CUs, else one workgroup per head (at 20x20 and

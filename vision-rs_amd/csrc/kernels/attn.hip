@@ -248,6 +248,201 @@ extern "C" __global__ __launch_bounds__(320) void vrs_psa_attn_bf16(vrs_attn_arg
 extern "C" __global__ __launch_bounds__(320) void vrs_psa_attn_f32(vrs_attn_args a) { attn_body<float, 5>(a); }
 
 // ---------------------------------------------------------------------------
+// Split-key attention, for few (image, head, query) blocks: the streamed kernel
+// gave a 20x20 map of 2 heads 10 workgroups that walk all keys (36 us in
+// float32), the resident one 2 workgroups per head.  Latency bounds these, so a
+// workgroup takes 16 queries and its KW waves share the keys: wave w the chunks
+// of 64 keys w, w + KW, ...  Each wave holds its own running max, sum and O^T;
+// they are combined through LDS at the end, in wave order.  K and V go from
+// global memory straight into MFMA operands, all loads of a chunk in flight
+// together: S^T = K Q^T has keys as rows (16 bytes of kd per lane); for O^T =
+// V^T P^T lane i of each 16 loads channels 4i..4i+3 of its keys, so operand dt
+// is channel 4i + dt and the row-major V needs no transpose in float32 (in
+// bfloat16 two keys' halves are paired by one v_perm each).
+// Measured, earlier kernel -> this (graph launches): float32 20x20, 2 heads x 1
+// 35.1 -> 8.3 us, 4 heads x 32 105 -> 62 us, 40x40, 4 heads x 8 300 -> 168 us;
+// bfloat16 20x20, 4 heads x 1 13.9 -> 5.5 us (floor of a launch 3.5), x 8 14.7
+// -> 12.6 us, x 16 15.3 -> 20.6 us (resident kernel kept); 40x40, 4 heads x 1
+// 38.5 -> 16.9 us, x 8 68 -> 85 us (streamed kernel kept).  Every workgroup
+// reads all of its head's K and V, from L2: that is what the larger problems
+// pay for.  Float32 error against float64 7.5e-8 (8.1e-8 before).
+namespace {
+template <typename T, int KW>
+__device__ __forceinline__ void attn_split_body(const vrs_attn_args& a) {
+  using E = Elt<T>;
+  using G = typename E::group;
+  constexpr int ES = (int)sizeof(T);
+  using VQ = typename std::conditional<ES == 2, u32x2_t, u32x4_t>::type;   // 4 channels of one key
+  constexpr int OL = VD + 4;                        // O row in LDS (padded)
+  __shared__ __attribute__((aligned(16))) float sO[KW][16 * OL];
+  __shared__ float sM[KW][16], sL[KW][16];
+  const int N = a.H * a.W;
+  const int logical = xcd_remap(blockIdx.x, gridDim.x);
+  const int qblk = logical % a.q_blocks;
+  const int bh = logical / a.q_blocks;
+  const int h = bh % a.heads, b = bh / a.heads;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  const int64_t img = (int64_t)b * N;
+  const int hc = h * (2 * KD + VD), q0 = qblk * 16;
+  // this image's rows (under 2 GiB, host); byte offset of channel c of pixel n
+  // (past the map: zeros)
+  const T* qkv = reinterpret_cast<const T*>(a.qkv) + img * a.qkv_pitch + hc;
+  const __amdgpu_buffer_rsrc_t rq = make_rsrc(qkv, ((N - 1) * a.qkv_pitch + 2 * KD + VD) * ES);
+  auto off = [&](int n, int c) { return n < N ? (uint32_t)(n * a.qkv_pitch + c) * (uint32_t)ES : kOOB; };
+
+  const G qf = E::bload(rq, off(q0 + i, g * 8), 0);
+  f32x4_t o[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) o[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_part = 0.f;
+  for (int kc = wave * KC; kc < N; kc += KW * KC) {
+    G kf[4];
+    VQ vv[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) kf[t] = E::bload(rq, off(kc + t * 16 + i, KD + g * 8), 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t vo = off(kc + t * 16 + g * 4 + r, 2 * KD + 4 * i);
+        if constexpr (ES == 2) vv[t][r] = __builtin_amdgcn_raw_buffer_load_b64(rq, vo, 0, 0);
+        else vv[t][r] = __builtin_amdgcn_raw_buffer_load_b128(rq, vo, 0, 0);
+      }
+    f32x4_t s[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) s[t] = mfma_k32(kf[t], qf, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+    float cmax = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (kc + t * 16 + g * 4 + r >= N) s[t][r] = -INFINITY;
+        cmax = fmaxf(cmax, s[t][r]);
+      }
+    cmax = xor_max<16>(cmax);
+    cmax = xor_max<32>(cmax);
+    // running max in log2 units; p = exp2(s c - m) is one FMA and an exponential,
+    // so the only rounding of a score's exponent is that of the difference
+    const float m_new = fmaxf(m_run, cmax * a.scale_log2e);   // finite: the chunk's first key exists
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    m_run = m_new;
+    float psum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], a.scale_log2e, -m_new));
+        if constexpr (ES == 2) p = bf2f(f2bf(p));   // the sum of exactly what P V consumes
+        s[t][r] = p;
+        psum += p;
+      }
+    l_part = l_part * alpha + psum;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) o[t] *= alpha;
+    if constexpr (ES == 2) {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {   // keys of tiles 2kk and 2kk + 1: g*4..g*4+3 of each
+        const f32x4_t s0 = s[2 * kk], s1 = s[2 * kk + 1];
+        G pf;
+        pf.v = (u32x4_t){pack_bf16x2(s0[0], s0[1]), pack_bf16x2(s0[2], s0[3]), pack_bf16x2(s1[0], s1[1]),
+                         pack_bf16x2(s1[2], s1[3])};
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          // halves dt & 1 of dword dt >> 1 of two keys
+          const uint32_t sel = (dt & 1) ? 0x07060302u : 0x05040100u;
+          G vf;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const VQ &x0 = vv[2 * kk + (w >> 1)][2 * (w & 1)], &x1 = vv[2 * kk + (w >> 1)][2 * (w & 1) + 1];
+            vf.v[w] = __builtin_amdgcn_perm(x1[dt >> 1], x0[dt >> 1], sel);
+          }
+          o[dt] = mfma_k32(vf, pf, o[dt]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)      // the step's 4 keys: g*4 + r of tile t
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt)
+            o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vv[t][r][dt % (int)(sizeof(VQ) / 4)]), s[t][r],
+                                                         o[dt], 0, 0, 0);
+    }
+  }
+  float l_tot = xor_sum<16>(l_part);
+  l_tot = xor_sum<32>(l_tot);
+  if (g == 0) {
+    sM[wave][i] = m_run;      // -inf and 0 for a wave without keys
+    sL[wave][i] = l_tot;
+  }
+  // accumulator register rr of o[dt]: channel 16 g + 4 rr + dt of query i
+#pragma unroll
+  for (int rr = 0; rr < 4; ++rr)
+    *reinterpret_cast<f32x4_t*>(&sO[wave][i * OL + 16 * g + 4 * rr]) = (f32x4_t){o[0][rr], o[1][rr], o[2][rr], o[3][rr]};
+
+  // this thread finishes channels d0..d0+PER-1 of query ql: the PE's nine taps
+  // (depthwise 3x3 on V, pad 1) are loaded before the barrier
+  constexpr int PER = 16 * VD / (KW * 64);
+  constexpr int PD = PER * ES / 4;                   // dwords
+  using P = uint32_t __attribute__((ext_vector_type(PD)));
+  const int ql = tid / (VD / PER), d0 = tid % (VD / PER) * PER;
+  const int qn = q0 + ql;
+  const int qy = qn / a.W, qx = qn - qy * a.W;
+  const int C = a.heads * VD, c0 = h * VD + d0;
+  const T* wpe = reinterpret_cast<const T*>(a.pe_w);
+  P tv[9], tw[9];
+#pragma unroll
+  for (int t = 0; t < 9; ++t) {
+    const int yy = qy + t / 3 - 1, xx = qx + t % 3 - 1;
+    const bool ok = qn < N && (unsigned)yy < (unsigned)a.H && (unsigned)xx < (unsigned)a.W;
+    const int pix = ok ? yy * a.W + xx : 0;
+    tv[t] = *reinterpret_cast<const P*>(qkv + (int64_t)pix * a.qkv_pitch + 2 * KD + d0);
+    tw[t] = *reinterpret_cast<const P*>(wpe + t * C + c0);
+    if (!ok) tv[t] = (P)(0u), tw[t] = (P)(0u);
+  }
+  __syncthreads();
+  if (qn >= N) return;
+  float m_all = sM[0][ql];
+#pragma unroll
+  for (int w = 1; w < KW; ++w) m_all = fmaxf(m_all, sM[w][ql]);
+  float l_all = 0.f, acc[PER];
+#pragma unroll
+  for (int e = 0; e < PER; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int w = 0; w < KW; ++w) {
+    const float f = __builtin_amdgcn_exp2f(sM[w][ql] - m_all);   // 0 for a wave without keys
+    l_all += f * sL[w][ql];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) acc[e] += f * sO[w][ql * OL + d0 + e];
+  }
+  const float inv = 1.f / l_all;
+  float res[PER];
+  auto val = [&](const P& v, int e) {
+    if constexpr (ES == 2) return __uint_as_float((e & 1) ? (v[e >> 1] & 0xffff0000u) : (v[e >> 1] << 16));
+    else return __uint_as_float(v[e]);
+  };
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    float pe = 0.f;
+#pragma unroll
+    for (int t = 0; t < 9; ++t) pe += val(tw[t], e) * val(tv[t], e);
+    res[e] = acc[e] * inv + pe * a.pe_scale[c0 + e] + a.pe_shift[c0 + e];
+  }
+  P ov;
+#pragma unroll
+  for (int d = 0; d < PD; ++d) ov[d] = ES == 2 ? pack_bf16x2(res[(2 * d) % PER], res[(2 * d + 1) % PER]) : __float_as_uint(res[d % PER]);
+  *reinterpret_cast<P*>(reinterpret_cast<T*>(a.out) + (img + qn) * a.out_pitch + h * VD + d0) = ov;
+}
+}  // namespace
+
+extern "C" __global__ __launch_bounds__(256, 2) void vrs_psa_attn_s4_bf16(vrs_attn_args a) { attn_split_body<bf16_t, 4>(a); }
+extern "C" __global__ __launch_bounds__(512, 2) void vrs_psa_attn_s8_bf16(vrs_attn_args a) { attn_split_body<bf16_t, 8>(a); }
+extern "C" __global__ __launch_bounds__(256, 2) void vrs_psa_attn_s4_f32(vrs_attn_args a) { attn_split_body<float, 4>(a); }
+extern "C" __global__ __launch_bounds__(512, 2) void vrs_psa_attn_s8_f32(vrs_attn_args a) { attn_split_body<float, 8>(a); }
+
+// ---------------------------------------------------------------------------
 // Resident-head attention, bfloat16, N <= 512 keys (every PSA map of YOLO26 at
 // 640: 20x20).  Workgroup = (b, h, QT query tiles of 32), one wave per query
 // tile.  The head's K ([key][kd], 80-byte rows) and V ([key][d], 128-byte rows,

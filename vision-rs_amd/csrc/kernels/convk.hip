@@ -15,8 +15,8 @@
 // MFMA fragments directly, a row per lane, was bound by the 64 lines each load
 // touches), three steps in flight in registers, through LDS rows that no
 // other wave touches, so the loop has no barrier.  At the end the KW partial
-// tiles are summed through LDS in wave order (fixed: the result does not
-// depend on timing).  KW = 1 (short K): four waves take four neighbouring
+// tiles are summed through LDS in a fixed order (the result does not depend on
+// timing).  KW = 1 (short K): four waves take four neighbouring
 // pixel tiles and nothing is summed.
 // Measured (graph launches, of which an empty one takes about 3.5 us), best
 // earlier tile -> this kernel: float32 3x3 128->128 at 40x40 x 1 58 -> 11.7 us
@@ -267,7 +267,7 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
     for (int i = 0; i < NQ; ++i)
       finish((f32x4_t){acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]}, i, sc[i], sh[i]);
   } else {
-    // each wave's partial tile over its own staging rows, summed in wave order
+    // each wave's partial tile over its own staging rows, summed in a fixed order
     static_assert(NQ * 64 * 16 <= 2 * TS * ROW, "partial tile fits the staging rows");
     f32x4_t* part = reinterpret_cast<f32x4_t*>(sa);
 #pragma unroll
@@ -275,10 +275,15 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
       part[i * 64 + lane] = (f32x4_t){acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]};
     __syncthreads();
     if (finishes) {
-      f32x4_t s = reinterpret_cast<const f32x4_t*>(lds[0])[tid];
+      // pairwise: half the rounding steps of a running sum
+      f32x4_t s[KW];
 #pragma unroll
-      for (int w = 1; w < KW; ++w) s += reinterpret_cast<const f32x4_t*>(lds[w])[tid];
-      finish(s, qd0, sc[0], sh[0]);
+      for (int w = 0; w < KW; ++w) s[w] = reinterpret_cast<const f32x4_t*>(lds[w])[tid];
+#pragma unroll
+      for (int d = 1; d < KW; d *= 2)
+#pragma unroll
+        for (int w = 0; w + d < KW; w += 2 * d) s[w] += s[w + d];
+      finish(s[0], qd0, sc[0], sh[0]);
     }
   }
 }
