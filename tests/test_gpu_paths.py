@@ -176,3 +176,67 @@ def test_attention_paths(dtype, b, heads, h, w):
     err = float((out[..., 4:c + 4].double() - ref).abs().max() / ref.square().mean().sqrt())
     assert err < (1e-5 if dtype == vrs.F32 else 4e-2), err
     assert torch.all(out[..., :4] == 7.0) and torch.all(out[..., c + 4:] == 7.0)
+
+
+@pytest.mark.parametrize("h,w,nc,thr,max_det", [
+    (64, 96, 5, 0.25, 10),         # 126 anchors: all kept ones sorted
+    (96, 160, 80, 0.001, 300),     # 315 anchors (odd)
+    (128, 128, 1, 0.0, 1024),      # one class, every anchor kept
+    (640, 640, 9, 0.001, 300),     # 8400 anchors: radix select
+    (1024, 1056, 3, 0.001, 1000),  # 22176 anchors: more than the registers hold
+])
+def test_detect_postprocess_paths(h, w, nc, thr, max_det):
+    """Near-equal, saturated, underflowing, infinite and NaN logits: class,
+    score and order as the plain loop over sigmoids gives them, bit for bit."""
+    import torch
+    rng = np.random.default_rng([h, w, nc])
+    strides = (8, 16, 32)
+    sizes = [(h // s) * (w // s) for s in strides]
+    A, n = sum(sizes), 2
+    lg = rng.normal(-3, 2, (n, nc, A)).astype(np.float32)
+    kind = rng.integers(0, 12, (n, A))
+    base = rng.normal(-2, 3, (n, 1, A)).astype(np.float32)
+    lg = np.where((kind == 0)[:, None], base + rng.integers(0, 3, lg.shape).astype(np.float32) * np.float32(1e-7), lg)
+    lg = np.where((kind == 1)[:, None], base + rng.uniform(0, 2e-3, lg.shape).astype(np.float32), lg)
+    lg = np.where((kind == 2)[:, None], rng.uniform(4.9, 30, lg.shape).astype(np.float32), lg)
+    lg = np.where((kind == 3)[:, None], rng.uniform(-110, -79, lg.shape).astype(np.float32), lg)
+    odd = rng.choice(np.array([np.nan, np.inf, -np.inf, 0.0, -0.0], np.float32), lg.shape)
+    lg = np.where((kind == 4)[:, None] & (rng.integers(0, 3, lg.shape) == 0), odd, lg).astype(np.float32)
+    boxes = rng.uniform(0, 5, (n, 4, A)).astype(np.float32)
+
+    def flat(t):   # per-scale blocks, channel-major inside each
+        parts, at = [], 0
+        for sz in sizes:
+            parts.append(t[:, :, at:at + sz].reshape(n, -1))
+            at += sz
+        return torch.from_numpy(np.concatenate(parts, 1)).cuda()
+
+    count, score, cls, anchor, xywh = ctx().detect_postprocess(flat(boxes), flat(lg), nc, h, w, strides, thr, max_det)
+    p = 1.0 / (1.0 + torch.exp(-torch.from_numpy(lg).cuda()))
+    best, bc = p[:, 0].clone(), torch.zeros(n, A, dtype=torch.int64, device="cuda")
+    for c in range(1, nc):   # Iterator::max_by with partial_cmp().unwrap_or(Equal)
+        take = ~(best > p[:, c])
+        best = torch.where(take, p[:, c], best)
+        bc = torch.where(take, torch.full_like(bc, c), bc)
+    best, bc = best.cpu().numpy(), bc.cpu().numpy()
+    for b in range(n):
+        kept = np.flatnonzero(best[b] >= np.float32(thr))
+        order = kept[np.argsort(-best[b][kept], kind="stable")][:max_det]
+        k = int(count[b])
+        assert k == len(order)
+        assert np.array_equal(anchor[b, :k].cpu().numpy(), order)
+        assert np.array_equal(score[b, :k].cpu().numpy().view(np.uint32), best[b][order].view(np.uint32))
+        assert np.array_equal(cls[b, :k].cpu().numpy(), bc[b][order])
+        assert torch.all(anchor[b, k:] == -1) and torch.all(score[b, k:] == 0) and torch.all(cls[b, k:] == -1)
+        a0, want = 0, []
+        for s, sz in zip(strides, sizes):
+            sel = [(i, a) for i, a in enumerate(order) if a0 <= a < a0 + sz]
+            for i, a in sel:
+                l, t, r, bo = boxes[b, :, a]
+                jx, jy = (a - a0) % (w // s), (a - a0) // (w // s)
+                want.append((i, (jx + 0.5) * s + s * (r - l) * 0.5, (jy + 0.5) * s + s * (bo - t) * 0.5, s * (l + r),
+                             s * (t + bo)))
+            a0 += sz
+        if k:
+            want = np.array(sorted(want), np.float64)[:, 1:]
+            assert np.max(np.abs(xywh[b, :k].cpu().numpy() - want)) < 1e-3 * 4   # float32 at up to 1100 pixels

@@ -1,24 +1,38 @@
 // Detect-head post-processing on gfx950.
 //
-// Stage 1 (one thread per anchor): LTRB -> xywh decode, sigmoid per class,
-// argmax, threshold -- the host loops of examples/yolo26.rs:1488-1528 with
-// the anchor grid of loss/anchor.rs:47-66.  The argmax follows Rust's
-// Iterator::max_by with partial_cmp().unwrap_or(Equal): the running best is
-// kept only if it compares Greater, so the last of equal maxima wins and a
-// NaN compares Equal.  A kept anchor gets the unique 64-bit key
-// (score_bits << 32) | (0xffffffff - anchor): ordering keys descending is the
-// stable descending sort of examples/yolo26.rs:1529 (equal scores keep
-// ascending anchor order); sigmoid scores are non-negative so their IEEE bits
-// order like the values.
+// Stage 1: LTRB -> xywh decode, sigmoid per class, argmax, threshold -- the
+// host loops of examples/yolo26.rs:1488-1528 with the anchor grid of
+// loss/anchor.rs:47-66.  The argmax follows Rust's Iterator::max_by with
+// partial_cmp().unwrap_or(Equal): the running best is kept only if it compares
+// Greater, so the last of equal maxima wins and a NaN compares Equal.  A kept
+// anchor gets the unique 64-bit key (score_bits << 32) | (0xffffffff -
+// anchor): ordering keys descending is the stable descending sort of
+// examples/yolo26.rs:1529 (equal scores keep ascending anchor order); sigmoid
+// scores are non-negative so their IEEE bits order like the values.
 //
 // Stage 2 (one workgroup per image): exact top-k (k = min(count, max_det)).
 // With at most TOPK_MAX kept anchors every key is gathered into LDS and
 // bitonic-sorted.  Otherwise a most-significant-digit radix select raises a
-// threshold 8 bits at a time and stops as soon as the keys at or above it
-// fit the LDS buffer (at the latest after the 8th digit, when the threshold
+// threshold 11 bits at a time and stops as soon as the keys at or above it
+// fit the LDS buffer (at the latest after the 6th digit, when the threshold
 // is the k-th largest key itself); those keys are gathered and sorted.
 #include "common.h"
 
+// four floats at any dword address (the workspace's boxes start after 8-byte keys)
+typedef float f32x4_any __attribute__((vector_size(16), aligned(4)));
+
+// Stage 1 reads the logits once (bs64 640, 80 classes: 172 MB); with a sigmoid
+// per logit and a load waited for at a time it took 61 us.  Only the largest
+// logit's sigmoid is computed: the sigmoid's rounding (a few ulp) can only
+// reorder logits within 2e-5 of each other when they are negative (its relative
+// slope is at least 1/2 there: 80 ulp), within 1e-3 up to 5 (at least 1/150: 50
+// ulp), any at or above 5, where it flattens to 1, and any below -80, where it
+// underflows.  An anchor whose second largest logit is that near, or that has
+// a NaN, goes through the classes again in order (those near enough; all of
+// them for NaN and underflow), so the class and score are those of the plain
+// loop, bit for bit.  One anchor per
+// thread, eight classes in flight: 34.3 us = 5.2 TB/s, a large copy's rate (two
+// and four anchors per thread 34.5 and 37.4 us).
 extern "C" __global__ __launch_bounds__(256) void vrs_detect_stage1(vrs_det1_args a) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (int64_t)a.B * a.A) return;
@@ -27,128 +41,197 @@ extern "C" __global__ __launch_bounds__(256) void vrs_detect_stage1(vrs_det1_arg
   while (s + 1 < a.nscales && ai >= a.a_base[s + 1]) ++s;
   const int as = (s + 1 < a.nscales ? a.a_base[s + 1] : a.A) - a.a_base[s];
   const int j = ai - a.a_base[s];
+  const float* sc = a.scores + (int64_t)b * a.nc * a.A + (int64_t)a.nc * a.a_base[s] + j;
+
+  float xm = sc[0], sec = -INFINITY;   // largest and second largest logit
+  int bc = 0;
+  bool nan = xm != xm;
+  auto see = [&](float x, int c) {
+    sec = fmaxf(sec, fminf(x, xm));
+    bc = x >= xm ? c : bc;
+    xm = fmaxf(xm, x);
+    nan |= x != x;
+  };
+  int c = 1;
+  for (; c + 8 <= a.nc; c += 8) {
+    float x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = sc[(int64_t)(c + u) * as];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) see(x[u], c + u);
+  }
+  for (; c < a.nc; ++c) see(sc[(int64_t)c * as], c);
+
+  const float near = fminf(xm - (xm < 0.0f ? 2e-5f : 1e-3f), 5.0f);
+  const bool all = nan || xm < -80.0f;
+  float best;
+  if (all || sec >= near) {
+    best = -1.0f;
+    for (int c0 = 0; c0 < a.nc; c0 += 8) {
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = sc[(int64_t)min(c0 + u, a.nc - 1) * as];
+      for (int u = 0; u < 8 && c0 + u < a.nc; ++u) {
+        if (!all && x[u] < near) continue;
+        const float p = 1.0f / (1.0f + expf(-x[u]));
+        if (!(best > p)) { best = p; bc = c0 + u; }
+      }
+    }
+  } else {
+    best = 1.0f / (1.0f + expf(-xm));
+  }
+  const bool keep = best >= a.thr;
+  a.keys[i] = keep ? (((uint64_t)__float_as_uint(best)) << 32) | (uint64_t)(0xffffffffu - (uint32_t)ai) : 0ull;
+  if (!keep) return;   // nothing reads the other anchors' boxes and classes
   const float st = a.stride[s];
   const float* bb = a.boxes + (int64_t)b * 4 * a.A + 4 * (int64_t)a.a_base[s];
   const float l = bb[j], t = bb[as + j], r = bb[2 * as + j], bo = bb[3 * as + j];
   const float cx = ((float)(j % a.fw[s]) + 0.5f) * st;
   const float cy = ((float)(j / a.fw[s]) + 0.5f) * st;
-  float* xy = a.xywh + i * 4;
-  xy[0] = cx + st * (r - l) * 0.5f;
-  xy[1] = cy + st * (bo - t) * 0.5f;
-  xy[2] = st * (l + r);
-  xy[3] = st * (t + bo);
-
-  const float* sc = a.scores + (int64_t)b * a.nc * a.A + (int64_t)a.nc * a.a_base[s] + j;
-  float best = 1.0f / (1.0f + expf(-sc[0]));
-  int bc = 0;
-  for (int c = 1; c < a.nc; ++c) {
-    const float v = 1.0f / (1.0f + expf(-sc[(int64_t)c * as]));
-    if (!(best > v)) { best = v; bc = c; }
-  }
+  *reinterpret_cast<f32x4_any*>(a.xywh + i * 4) =
+      (f32x4_any){cx + st * (r - l) * 0.5f, cy + st * (bo - t) * 0.5f, st * (l + r), st * (t + bo)};
   a.cls[i] = bc;
-  a.keys[i] = (best >= a.thr) ? (((uint64_t)__float_as_uint(best)) << 32) | (uint64_t)(0xffffffffu - (uint32_t)ai)
-                              : 0ull;
 }
 
+// One workgroup per image, 64 of them at bs64: the time is its chain of
+// dependent steps.  The keys stay in registers (16 per thread; images of more
+// than 16384 anchors read the rest again per digit); a digit is 11 bits (16
+// bins per octave of the score: 8-bit digits put most keys into two bins, whose
+// LDS atomics then queue up) and its bin is found by a parallel scan (one
+// thread walking 256 bins took 10 us); the sort keeps one key per thread and
+// crosses lanes inside a wave.  39.5 -> 15.5 us at 8400 anchors, nearly
+// all kept (threshold 0.001).
 namespace {
 constexpr int TOPK_MAX = 1024;
+constexpr int KEY_REGS = 16;
+constexpr int DIGIT = 11, BINS = 1 << DIGIT;
 }
 
 extern "C" __global__ __launch_bounds__(1024) void vrs_detect_stage2(vrs_det2_args a) {
-  __shared__ uint32_t hist[256];
+  __shared__ uint32_t hist[BINS];
   __shared__ uint64_t sel[TOPK_MAX];
-  __shared__ uint32_t s_count, s_nsel, s_digit, s_krem, s_ntop;
-  const int b = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+  __shared__ uint32_t s_wave[16], s_nsel, s_digit, s_krem, s_ntop;
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint64_t* keys = a.keys + (int64_t)b * a.A;
 
-  if (tid == 0) { s_count = 0; s_nsel = 0; }
-  __syncthreads();
+  uint64_t reg[KEY_REGS];
+#pragma unroll
+  for (int r = 0; r < KEY_REGS; ++r) reg[r] = tid + r * 1024 < a.A ? keys[tid + r * 1024] : 0ull;
+  auto each_key = [&](auto f) {   // whole waves together (f may use ballots)
+#pragma unroll
+    for (int r = 0; r < KEY_REGS; ++r)
+      if (r * 1024 < a.A) f(reg[r]);
+    for (int i0 = KEY_REGS * 1024; i0 < a.A; i0 += 1024) f(i0 + tid < a.A ? keys[i0 + tid] : 0ull);
+  };
+  // inclusive sum over the workgroup's threads; two barriers
+  auto block_scan = [&](uint32_t v) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t u = __shfl_up(v, d);
+      if (lane >= d) v += u;
+    }
+    if (lane == 63) s_wave[wave] = v;
+    __syncthreads();
+    uint32_t before = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) before += w < wave ? s_wave[w] : 0u;
+    __syncthreads();
+    return v + before;
+  };
+
   uint32_t local = 0;
-  for (int i = tid; i < a.A; i += nt) local += keys[i] != 0ull;
-  atomicAdd(&s_count, local);
+  each_key([&](uint64_t key) { local += key != 0ull; });
+  const uint32_t upto = block_scan(local);
+  if (tid == 1023) s_krem = upto;
+  if (tid == 0) s_nsel = 0;
   __syncthreads();
-  const uint32_t count = s_count;
+  const uint32_t count = s_krem;
   const uint32_t k = count < (uint32_t)a.max_det ? count : (uint32_t)a.max_det;
 
   // gather threshold: every nonzero key when they all fit the buffer
   uint64_t thr_key = 1ull;
   if (count > (uint32_t)TOPK_MAX && k > 0) {
     uint64_t prefix = 0, pmask = 0;
-    if (tid == 0) s_krem = k;
-    for (int shift = 56; shift >= 0; shift -= 8) {
-      for (int i = tid; i < 256; i += nt) hist[i] = 0;
+    uint32_t krem = k;
+    // scores are at most 1.0f: bits 62 and 63 of a key are zero
+    for (int shift = 62 - DIGIT; ; shift = shift > DIGIT ? shift - DIGIT : 0) {
+      hist[tid] = 0;
+      hist[tid + 1024] = 0;
       __syncthreads();
-      for (int i = tid; i < a.A; i += nt) {
-        const uint64_t key = keys[i];
-        if (key != 0ull && (key & pmask) == prefix) atomicAdd(&hist[(key >> shift) & 255u], 1u);
-      }
+      each_key([&](uint64_t key) {
+        if (key != 0ull && (key & pmask) == prefix) atomicAdd(&hist[(uint32_t)(key >> shift) & (BINS - 1)], 1u);
+      });
       __syncthreads();
-      if (tid == 0) {
-        uint32_t cum = 0, krem = s_krem;
-        int d = 255;
-        for (; d > 0; --d) {
-          if (cum + hist[d] >= krem) break;
-          cum += hist[d];
-        }
-        s_digit = (uint32_t)d;
-        s_krem = krem - cum;
+      // thread t scans bins BINS-1-2t and BINS-2-2t, from the top down
+      const uint32_t hi = hist[BINS - 1 - 2 * tid], lo = hist[BINS - 2 - 2 * tid];
+      const uint32_t incl = block_scan(hi + lo), excl = incl - hi - lo;
+      if (excl < krem && krem <= incl) {   // one thread: the bin of the krem-th key
+        const bool top = krem <= excl + hi;
+        const uint32_t above = top ? excl : excl + hi;
+        s_digit = (uint32_t)(BINS - 1 - 2 * tid) - (top ? 0u : 1u);
+        s_krem = krem - above;
         // keys whose digits so far are >= the new prefix: above it at the
-        // earlier digits (k - krem), in the higher bins of this one (cum),
-        // and in bin d
-        s_ntop = (k - krem) + cum + hist[d];
+        // earlier digits (k - krem), in the higher bins of this one and in it
+        s_ntop = (k - krem) + above + (top ? hi : lo);
       }
       __syncthreads();
+      krem = s_krem;
       prefix |= ((uint64_t)s_digit) << shift;
-      pmask |= 255ull << shift;
+      pmask |= ((uint64_t)(BINS - 1)) << shift;
       const bool fits = s_ntop <= (uint32_t)TOPK_MAX;
       __syncthreads();
-      if (fits) break;
+      if (fits || shift == 0) break;
     }
     // lower bits zero: the keys >= prefix are exactly those counted in s_ntop,
     // and they include the k largest
     thr_key = prefix;
   }
 
-  for (int i = tid; i < TOPK_MAX; i += nt) sel[i] = 0ull;
+  sel[tid] = 0ull;
   __syncthreads();
   if (k > 0)
-    for (int i = tid; i < a.A; i += nt) {
-      const uint64_t key = keys[i];
-      if (key != 0ull && key >= thr_key) {
-        const uint32_t slot = atomicAdd(&s_nsel, 1u);
-        if (slot < (uint32_t)TOPK_MAX) sel[slot] = key;
-      }
-    }
+    each_key([&](uint64_t key) {
+      const bool in = key != 0ull && key >= thr_key;
+      const uint64_t m = __ballot(in);
+      uint32_t base = 0;
+      if (lane == 0 && m) base = atomicAdd(&s_nsel, (uint32_t)__popcll(m));
+      base = __shfl(base, 0);
+      const uint32_t slot = base + (uint32_t)__popcll(m & ((1ull << lane) - 1));
+      if (in && slot < (uint32_t)TOPK_MAX) sel[slot] = key;
+    });
   __syncthreads();
   // sort the smallest power of two of slots holding every gathered key
   const uint32_t nsel = s_nsel < (uint32_t)TOPK_MAX ? s_nsel : (uint32_t)TOPK_MAX;
   int P = 2;
   while ((uint32_t)P < nsel) P <<= 1;
 
-  // bitonic sort, descending, over P slots (zeros sink to the end)
+  // bitonic sort, descending, over P slots (zeros sink to the end): thread t
+  // holds slot t; partners in the same wave by shuffle, others through LDS
+  uint64_t el = sel[tid];
   for (int size = 2; size <= P; size <<= 1)
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = tid; i < P; i += nt) {
-        const int j = i ^ stride;
-        if (j > i) {
-          const bool desc = (i & size) == 0;
-          const uint64_t x = sel[i], y = sel[j];
-          if (desc ? (x < y) : (x > y)) { sel[i] = y; sel[j] = x; }
-        }
+      uint64_t y;
+      if (stride >= 64) {
+        __syncthreads();
+        sel[tid] = el;
+        __syncthreads();
+        y = sel[tid ^ stride];
+      } else {
+        y = __shfl_xor((unsigned long long)el, stride);
       }
-      __syncthreads();
+      const bool larger = ((tid & stride) == 0) == ((tid & size) == 0);
+      el = (el > y) == larger ? el : y;
     }
 
   if (tid == 0) a.count[b] = (int32_t)k;
-  for (int i = tid; i < a.max_det; i += nt) {
-    const int64_t o = (int64_t)b * a.max_det + i;
-    if ((uint32_t)i < k) {
-      const uint64_t key = sel[i];
-      const int anchor = (int)(0xffffffffu - (uint32_t)(key & 0xffffffffull));
-      a.out_score[o] = __uint_as_float((uint32_t)(key >> 32));
+  if (tid < a.max_det) {   // max_det <= 1024 (host)
+    const int64_t o = (int64_t)b * a.max_det + tid;
+    if ((uint32_t)tid < k) {
+      const int anchor = (int)(0xffffffffu - (uint32_t)(el & 0xffffffffull));
+      a.out_score[o] = __uint_as_float((uint32_t)(el >> 32));
       a.out_anchor[o] = anchor;
       a.out_cls[o] = a.cls[(int64_t)b * a.A + anchor];
-      const float* xy = a.xywh + ((int64_t)b * a.A + anchor) * 4;
+      const f32x4_any xy = *reinterpret_cast<const f32x4_any*>(a.xywh + ((int64_t)b * a.A + anchor) * 4);
 #pragma unroll
       for (int q = 0; q < 4; ++q) a.out_xywh[o * 4 + q] = xy[q];
     } else {
