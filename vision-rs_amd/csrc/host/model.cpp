@@ -136,6 +136,7 @@ struct vrs_model {
   std::vector<LaunchIO> io;      // per launch: what it reads and writes
   std::vector<int> conv_launch;  // per conv: index of its kernel launch (-1: none)
   int streams = 3;               // capture concurrency: the trunk plus side streams for the Detect chains
+  bool streams_set = false;      // by the caller (else a small forward captures one chain)
   std::vector<hipStream_t> side; // extra capture streams (default priority)
   const float* prep_x = nullptr;
   std::vector<float*> prep_outs;
@@ -1647,7 +1648,16 @@ int vrs_model_capture(vrs_model* m, const float* x, float* const* outputs, void*
   // sibling branch of the trunk as well, and sending every chain to a side
   // stream of its own, were slower still.)
   const int n = (int)m->launches.size();
-  const int K = std::max(1, std::min(m->streams, 8));
+  // A small forward stays one chain unless the caller asked for streams: its
+  // launches are short, and each edge between streams costs more than running
+  // beside the trunk gains (YOLO26n float32 batch 1 573 us on one stream, 651 on
+  // three; YOLO26m bf16 batch 1 690 vs 815, batch 16 2292 vs 2191; YOLO26s bf16
+  // batch 8, about 1 ms, the same).  Small: under 0.75 ms of work at the rates
+  // the kernels reach (600 and 60 TFLOP/s, 4 TB/s).
+  double work = 0.0;
+  for (const Launch& l : m->launches)
+    work += std::max(l.flops / (act_dt(m) == VRS_F32 ? 60e12 : 600e12), l.bytes / 4e12);
+  const int K = !m->streams_set && work < 0.75e-3 ? 1 : std::max(1, std::min(m->streams, 8));
   auto conflict = [](const LaunchIO& a, const LaunchIO& b) {   // a after b
     auto ov = [](const Access& x, const Access& y) { return x.res == y.res && x.c0 < y.c1 && y.c0 < x.c1; };
     for (const Access& w : a.wr) {
@@ -1764,6 +1774,7 @@ int vrs_model_set_streams(vrs_model* m, int32_t streams) {
   if (!m) return fail(VRS_EINVAL, "null model");
   if (streams < 1 || streams > 8) return fail(VRS_EINVAL, "vrs_model_set_streams: %d (1..8)", streams);
   m->streams = streams;
+  m->streams_set = true;
   return VRS_OK;
 }
 
