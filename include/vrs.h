@@ -128,8 +128,8 @@ typedef struct {
  * vrs_conv_pointwise_pair launch; the first conv then has no launch and no
  * output of its own. */
 #define VRS_TILE_PWPAIR 13
-/* Split-K kernels for small problems (bf16 and float32, k up to 5, any
- * stride, fused upsample and flat outputs included): one 32x32 or 16x16 output
+/* Split-K kernels for small problems (bf16, float32, and VRS_FP8 with an e4m3
+ * input; k up to 5, any stride, fused upsample and flat outputs included): one 32x32 or 16x16 output
  * tile per workgroup, whose waves share the K range and sum their parts in a
  * fixed order.  OR one of VRS_TILE_SPLIT(n) for the number of waves sharing K:
  * 1 (16x16 only: four neighbouring tiles per workgroup), 4 or 8; none: by the

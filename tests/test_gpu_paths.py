@@ -240,3 +240,45 @@ def test_detect_postprocess_paths(h, w, nc, thr, max_det):
         if k:
             want = np.array(sorted(want), np.float64)[:, 1:]
             assert np.max(np.abs(xywh[b, :k].cpu().numpy() - want)) < 1e-3 * 4   # float32 at up to 1100 pixels
+
+
+@pytest.mark.parametrize("tile", SPLIT_TILES + [pytest.param(vrs.TILE_AUTO, id="auto")])
+@pytest.mark.parametrize("n,cin,h,w,cout,k,s,res,y8", [
+    (1, 64, 1, 1, 16, 1, 1, None, False),    # one pixel, half a step of K
+    (1, 64, 5, 7, 48, 3, 1, "e4m3", True),   # taps of half a step
+    (2, 128, 6, 5, 32, 3, 2, None, True),    # taps of one step
+    (1, 192, 4, 9, 80, 1, 1, "bf16", False),
+    (1, 512, 3, 3, 16, 3, 1, "bf16", True),  # deep K
+])
+def test_split_k_fp8(n, cin, h, w, cout, k, s, res, y8, tile):
+    """The same sums in another order as the 128x128 fp8 tile (which other tests
+    hold against the oracle): at most one rounding apart."""
+    import torch
+    torch.manual_seed(cin + cout)
+    x = (torch.randn(n, h, w, cin + 16, device="cuda") * 2).to(torch.float8_e4m3fn).view(torch.uint8)
+    rng = np.random.default_rng(cin)
+    q, ws = vrs.pack_conv_weight_fp8((rng.standard_normal((cout, cin, k, k)) * np.sqrt(2.0 / (cin * k * k))).astype(np.float32))
+    q, sc = torch.from_numpy(q).cuda(), torch.from_numpy(ws).cuda() * (torch.rand(cout, device="cuda") + 0.5)
+    sh = torch.randn(cout, device="cuda") * 0.2
+    ho, wo = (h - 1) // s + 1, (w - 1) // s + 1
+    rt = None
+    if res:
+        rt = torch.randn(n, ho, wo, cout + 16, device="cuda")
+        rt = rt.to(torch.float8_e4m3fn).view(torch.uint8) if res == "e4m3" else rt.bfloat16()
+    outs = []
+    for t in (vrs.TILE_128x128, tile):
+        y = torch.full((n, ho, wo, cout + 16), 0x55, dtype=torch.uint8, device="cuda")
+        y = y if y8 else y.bfloat16()
+        ctx().conv2d(vrs.nhwc(x, cin, 16), q, sc, sh, vrs.nhwc(y, cout, 16), k, s, 1, vrs.ACT_SILU,
+                     None if rt is None else vrs.nhwc(rt, cout, 16), vrs.FP8, tile=t, in_scale=1.0, x_e4m3=True,
+                     y_e4m3=y8, out_step=2.0 ** -5 if y8 else 0.0, res_e4m3=res == "e4m3",
+                     res_step=1.0 if res == "e4m3" else 0.0)
+        torch.cuda.synchronize()
+        assert torch.all(y[..., :16] == 0x55)
+        v = y[..., 16:].contiguous()
+        outs.append((v.view(torch.float8_e4m3fn) if y8 else v).double())
+    a, b = outs
+    step = 2.0 ** -3 if y8 else 2.0 ** -7     # one step of the output type, relative
+    small = (2.0 ** -9 if y8 else 1e-6) * float(a.abs().max())
+    assert torch.all((a - b).abs() <= step * a.abs() + small)
+    assert float((a != b).double().mean()) < 0.02   # float32 sums differ by 1e-6, roundings flip rarely

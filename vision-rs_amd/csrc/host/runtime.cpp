@@ -190,6 +190,11 @@ static int h3_strip_width(int w) {
   return 32;
 }
 
+// Input widths the fp8 weight-stationary 1x1 kernel is built for.
+static bool w1_fp8_cin(int cin) {
+  return cin == 128 || cin == 192 || cin == 256 || cin == 384 || cin == 512 || cin == 768;
+}
+
 // Predicted time of one conv on one tile (microseconds at 256 CUs), for the
 // automatic choice and to prune the autotuner's candidates:
 //   c0 + c1 * nk + c2 * wk * g + c3 * g + c4 * MB / 4,
@@ -201,8 +206,8 @@ static int h3_strip_width(int w) {
 // 1x1 and 3x3) on every tile of both types; median error 4-10 %.  Steps: '6'
 // 64-deep, '3' 32-deep, 'g' Cin not in whole steps, 'a' in whole steps.  The
 // tile it picks is 2 % over the best one (geometric mean), where the rule it
-// replaces (the widest tile that leaves two workgroups per CU) was 1.64x over
-// it in bfloat16 and 2.7x in float32.
+// replaces (the widest tile that leaves two workgroups per CU; fp8: 64x256 or
+// 128x128) was 1.64x over it in bfloat16, 2.7x in float32, 1.4x in fp8.
 struct TileCost { int dtype, tile; char steps; float c[5]; };
 static const TileCost kTileCost[] = {
     {VRS_BF16, VRS_TILE_128x128, 'g', {4.18, 0.543, 0.193, 1.62, 0.188}},
@@ -233,6 +238,22 @@ static const TileCost kTileCost[] = {
     {VRS_BF16, VRS_TILE_KW32 | VRS_TILE_SPLIT(8), 'g', {3.15, 0.54, 0.0928, 2.98, 0}},
     {VRS_BF16, VRS_TILE_W1_128, 0, {3.02, 0.287, 0.0197, 1.15, 0.248}},
     {VRS_BF16, VRS_TILE_W1_256, 0, {4.37, 0.335, 0, 1.06, 0.656}},
+    {VRS_FP8, VRS_TILE_128x128, '6', {5.07, 0.135, 0.0852, 1.78, 0.00507}},
+    {VRS_FP8, VRS_TILE_128x256, '6', {7.21, 0.192, 0.104, 5.13, 0.153}},
+    {VRS_FP8, VRS_TILE_256x128, '6', {7.41, 0.177, 0.131, 6.13, 0}},
+    {VRS_FP8, VRS_TILE_256x256, '6', {10.9, 0.259, 0.116, 6.61, 0.281}},
+    {VRS_FP8, VRS_TILE_64x256, '6', {5.49, 0.164, 0.0858, 1.95, 0.111}},
+    {VRS_FP8, VRS_TILE_KW16 | VRS_TILE_SPLIT(1), 'a', {3.09, 0.174, 0.12, 0.543, 0.204}},
+    {VRS_FP8, VRS_TILE_KW16 | VRS_TILE_SPLIT(1), 'g', {3.12, 0.218, 0.127, 0.524, 0}},
+    {VRS_FP8, VRS_TILE_KW16 | VRS_TILE_SPLIT(4), 'a', {2.94, 0.291, 0.0256, 0.526, 0}},
+    {VRS_FP8, VRS_TILE_KW16 | VRS_TILE_SPLIT(4), 'g', {3.04, 0.242, 0.031, 0.489, 0}},
+    {VRS_FP8, VRS_TILE_KW16 | VRS_TILE_SPLIT(8), 'a', {3.27, 0.327, 0.0275, 1.2, 0}},
+    {VRS_FP8, VRS_TILE_KW16 | VRS_TILE_SPLIT(8), 'g', {3.05, 0.304, 0.0308, 1.12, 0}},
+    {VRS_FP8, VRS_TILE_KW32 | VRS_TILE_SPLIT(4), 'a', {4.04, 0.337, 0.061, 1.18, 0}},
+    {VRS_FP8, VRS_TILE_KW32 | VRS_TILE_SPLIT(4), 'g', {3.81, 0.425, 0.0688, 1.09, 0}},
+    {VRS_FP8, VRS_TILE_KW32 | VRS_TILE_SPLIT(8), 'a', {4.65, 0.121, 0.0849, 3.07, 0}},
+    {VRS_FP8, VRS_TILE_KW32 | VRS_TILE_SPLIT(8), 'g', {3.75, 0.621, 0.0915, 2.92, 0}},
+    {VRS_FP8, VRS_TILE_W1_128, 0, {4.91, 0.182, 0.0212, 1.08, 0}},
     {VRS_F32, VRS_TILE_128x128, 'g', {3.9, 2.09, 1.54, 6.2, 0}},
     {VRS_F32, VRS_TILE_128x128, '3', {5.63, 1.85, 1.03, 4.79, 0.246}},
     {VRS_F32, VRS_TILE_32x256, 'g', {2.01, 1.53, 1.46, 4.64, 0}},
@@ -252,12 +273,27 @@ static const TileCost kTileCost[] = {
     {VRS_F32, VRS_TILE_KW32 | VRS_TILE_SPLIT(8), 'g', {3.16, 0.384, 0.163, 3.57, 0}},
 };
 
+// A tile's row for a type and step kind (null: not built), found once per
+// process: the choice prices some fifteen tiles per call.
+static const TileCost* tile_cost_row(int dtype, int tile, char steps) {
+  constexpr int kTilesMax = VRS_TILE_KW16 + 1;
+  struct Index {
+    const TileCost* row[3][kTilesMax][4][4] = {};   // [type][tile][split flag][step kind]
+    static int kind(char c) { return c == '6' || c == 'a' ? 1 : c == '3' ? 2 : c == 'g' ? 3 : 0; }
+    Index() {
+      for (const TileCost& t : kTileCost) row[t.dtype][t.tile & 0xff][t.tile >> 12][kind(t.steps)] = &t;
+    }
+  };
+  static const Index index;
+  return index.row[dtype][tile & 0xff][tile >> 12][Index::kind(steps)];
+}
+
 struct ConvShape { int cout, cin, k, dtype; int64_t m, in_px; };
 
 static double tile_cost(const ConvShape& s, int tile, int64_t h3_blocks, int num_cu) {
-  const int code = tile & 0xff, es = (int)elt_size(s.dtype);
+  const int code = tile & 0xff, es = s.dtype == VRS_FP8 ? 1 : (int)elt_size(s.dtype);
   const bool kw = code == VRS_TILE_KW32 || code == VRS_TILE_KW16;
-  const bool k64 = s.dtype == VRS_BF16 && s.cin % 64 == 0 && !(tile & VRS_TILE_K32) && code != VRS_TILE_32x256;
+  const bool k64 = s.dtype != VRS_F32 && s.cin % 64 == 0 && !(tile & VRS_TILE_K32) && code != VRS_TILE_32x256;
   char steps = kw ? (s.cin * es % 128 == 0 ? 'a' : 'g') : s.cin % 32 ? 'g' : k64 ? '6' : '3';
   int bm, bn;
   if (code == VRS_TILE_H3) bm = s.cout <= 32 ? 32 : 64, bn = 256, steps = 0;
@@ -266,29 +302,25 @@ static double tile_cost(const ConvShape& s, int tile, int64_t h3_blocks, int num
   else if (code == VRS_TILE_KW16) bm = 16, bn = (tile & VRS_TILE_SPLIT_MASK) == VRS_TILE_SPLIT(1) ? 64 : 16;
   else if (const TileInfo* t = tile_info(code)) bm = t->bm, bn = t->bn;
   else return 1e30;
-  const int key = kw ? tile : code;
-  for (const TileCost& t : kTileCost) {
-    if (t.dtype != s.dtype || t.tile != key || t.steps != steps) continue;
-    const int K = s.k * s.k * s.cin;
-    double nk, wk;
-    if (kw) {
-      const int split = (tile & VRS_TILE_SPLIT_MASK) == VRS_TILE_SPLIT(1)   ? 1
-                        : (tile & VRS_TILE_SPLIT_MASK) == VRS_TILE_SPLIT(4) ? 4
-                                                                            : 8;
-      wk = (K * es + 127) / 128;
-      nk = ((int)wk + split - 1) / split;
-    } else {
-      const int bk = k64 ? 64 : 32;
-      nk = wk = (double)((K + bk - 1) / bk) * (bk / 32);
-    }
-    const double blocks = code == VRS_TILE_H3 && h3_blocks > 0
-                              ? (double)h3_blocks
-                              : (double)((s.cout + bm - 1) / bm) * (double)((s.m + bn - 1) / bn);
-    const double g = blocks / (num_cu > 0 ? num_cu : 256);
-    const double mb = ((double)s.in_px * s.cin + (double)s.m * s.cout + (double)s.cout * K) * es * 1e-6;
-    return t.c[0] + t.c[1] * nk + t.c[2] * wk * g + t.c[3] * g + t.c[4] * mb / 4;
+  const TileCost* t = tile_cost_row(s.dtype, kw ? tile : code, steps);
+  if (!t) return 1e30;
+  const int K = s.k * s.k * s.cin;
+  double nk, wk;
+  if (kw) {
+    const int flag = tile & VRS_TILE_SPLIT_MASK;
+    const int split = flag == VRS_TILE_SPLIT(1) ? 1 : flag == VRS_TILE_SPLIT(4) ? 4 : 8;
+    wk = (K * es + 127) / 128;
+    nk = ((int)wk + split - 1) / split;
+  } else {
+    const int bk = k64 ? 64 : 32;
+    nk = wk = (double)((K + bk - 1) / bk) * (bk / 32);
   }
-  return 1e30;
+  const double blocks = code == VRS_TILE_H3 && h3_blocks > 0
+                            ? (double)h3_blocks
+                            : (double)((s.cout + bm - 1) / bm) * (double)((s.m + bn - 1) / bn);
+  const double g = blocks / (num_cu > 0 ? num_cu : 256);
+  const double mb = ((double)s.in_px * s.cin + (double)s.m * s.cout + (double)s.cout * K) * es * 1e-6;
+  return t->c[0] + t->c[1] * nk + t->c[2] * wk * g + t->c[3] * g + t->c[4] * mb / 4;
 }
 
 static const int kSplitTiles[] = {VRS_TILE_KW16 | VRS_TILE_SPLIT(1), VRS_TILE_KW16 | VRS_TILE_SPLIT(4),
@@ -304,9 +336,11 @@ static int auto_tile(const ConvSpec& cs, const vrs_conv_args& a, const vrs_nhwc&
   const bool staged = a.stage == 1 && !a.y_f32, g = a.Cin % 32 != 0;
   const int64_t want = 2ll * (num_cu > 0 ? num_cu : 256);
   auto blocks = [&](int bm, int bn) { return (int64_t)((s.cout + bm - 1) / bm) * ((s.m + bn - 1) / bn); };
+  const bool f8 = s.dtype == VRS_FP8;
   int best = VRS_TILE_128x128;
   if (!cs.up) {
-    if (s.cout <= 32) best = VRS_TILE_32x256;
+    if (f8) best = s.cout <= 64 ? VRS_TILE_64x256 : VRS_TILE_128x128;
+    else if (s.cout <= 32) best = VRS_TILE_32x256;
     else if (s.cout <= 64) best = VRS_TILE_64x256;
     else if (s.dtype == VRS_BF16 && !g && s.cout <= 128 && blocks(128, 256) >= want) best = VRS_TILE_128x256;
     else if (s.dtype == VRS_BF16 && !g && s.cout > 128 && blocks(256, 128) >= want) best = VRS_TILE_256x128;
@@ -320,12 +354,13 @@ static int auto_tile(const ConvSpec& cs, const vrs_conv_args& a, const vrs_nhwc&
     if (s.dtype == VRS_F32 && !ti.f32) continue;
     if (g && ti.code != VRS_TILE_128x128 && ti.code != VRS_TILE_64x256 && ti.code != VRS_TILE_32x256) continue;
     if (!ti.k32 && a.Cin % 64) continue;
+    if (f8 && (ti.code == VRS_TILE_32x256 || ti.code == VRS_TILE_64x64)) continue;
     if (cs.up && ti.code != VRS_TILE_128x128 && (ti.code != VRS_TILE_64x64 || (s.dtype == VRS_BF16 && a.Cin % 64)))
       continue;
     offer(ti.code);
   }
-  const int cps = 128 / (int)elt_size(s.dtype);
-  if (a.kh <= 5 && (!cs.up || (a.Cin % cps == 0 && a.c_split % cps == 0)))
+  const int cps = f8 ? 128 : 128 / (int)elt_size(s.dtype);
+  if (a.kh <= 5 && (!f8 || cs.x_f8) && (!cs.up || (a.Cin % cps == 0 && a.c_split % cps == 0)))
     for (int tile : kSplitTiles) offer(tile);
   const int tw = h3_strip_width(x.w);
   if (s.dtype == VRS_BF16 && a.kh == 3 && a.stride == 1 && !g && tw && !cs.up && staged && a.res_bytes >= 0 &&
@@ -336,16 +371,12 @@ static int auto_tile(const ConvSpec& cs, const vrs_conv_args& a, const vrs_nhwc&
     if (5 * runs * 256 <= 6ll * x.h * x.w)
       offer(VRS_TILE_H3, runs * x.n * ((s.cout + (s.cout <= 32 ? 31 : 63)) / (s.cout <= 32 ? 32 : 64)));
   }
+  if (f8 && a.kh == 1 && a.stride == 1 && !cs.up && w1_fp8_cin(a.Cin) && !a.res && staged) offer(VRS_TILE_W1_128);
   if (s.dtype == VRS_BF16 && a.kh == 1 && a.stride == 1 && !cs.up && a.Cin % 64 == 0 && !a.res && staged) {
     if (a.Cin <= 192) offer(VRS_TILE_W1_256);
     if (a.Cin <= 256 || a.Cin == 384) offer(VRS_TILE_W1_128);
   }
   return best;
-}
-
-// Input widths the fp8 weight-stationary 1x1 kernel is built for.
-static bool w1_fp8_cin(int cin) {
-  return cin == 128 || cin == 192 || cin == 256 || cin == 384 || cin == 512 || cin == 768;
 }
 
 std::vector<int> conv_tile_candidates(int cout, int cin, int dtype, int k, int stride, int w, int64_t m,
@@ -409,12 +440,13 @@ std::vector<int> conv_tile_candidates(int cout, int cin, int dtype, int k, int s
 // Split-K small-problem kernel (convk.hip) on prep_dense's argument block.
 static int prep_splitk(vrs_ctx* ctx, const ConvSpec& cs, int cout, vrs_conv_args& a, std::vector<Launch>& out) {
   const int ts = (cs.tile & 0xff) == VRS_TILE_KW32 ? 32 : 16;
-  if (cs.dtype != VRS_BF16 && cs.dtype != VRS_F32)
-    return fail(VRS_EUNSUPPORTED, "conv: the split-K tiles take bf16 or float32 (dtype %d)", cs.dtype);
+  const bool f8 = cs.dtype == VRS_FP8;
+  if (f8 && (!cs.x_f8 || a.Cin % 64))
+    return fail(VRS_EUNSUPPORTED, "conv fp8: the split-K tiles need an e4m3 input and Cin %% 64 == 0 (Cin=%d)", a.Cin);
   if (cs.tile & ~(0xff | VRS_TILE_SPLIT_MASK))
     return fail(VRS_EINVAL, "conv: tile code %d: the split-K tiles take only VRS_TILE_SPLIT flags", cs.tile);
   if (cs.k > 5) return fail(VRS_EUNSUPPORTED, "conv: the split-K tiles take k <= 5 (k=%d)", cs.k);
-  const int es = (int)elt_size(cs.dtype), cps = 128 / es;   // channels per 128-byte step
+  const int es = f8 ? 1 : (int)elt_size(cs.dtype), cps = 128 / es;   // channels per 128-byte step
   vrs_convk_args k{};
   k.gpt = a.Cin * es / 16;
   const bool aligned = a.Cin % cps == 0;
@@ -442,15 +474,16 @@ static int prep_splitk(vrs_ctx* ctx, const ConvSpec& cs, int cout, vrs_conv_args
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
   if (blocks >= (1ll << 31) / 1024) return fail(VRS_EBADSHAPE, "conv: grid too large for the split-K tile");
   char name[48];
-  snprintf(name, sizeof name, "vrs_conv_%s_s%d_w%d_%c", dsuffix(cs.dtype), ts, kw, aligned ? 'a' : 'g');
+  snprintf(name, sizeof name, "vrs_conv_%s_s%d_w%d_%c", f8 ? "fp8" : dsuffix(cs.dtype), ts, kw, aligned ? 'a' : 'g');
   hipFunction_t f;
   if (int rc = get_fn(ctx, name, &f)) return rc;
   out.push_back(make_launch(name, f, dim3((unsigned)blocks), dim3(64 * kw * nt), 0, k));
   const double cin = cs.cin_real > 0 ? cs.cin_real : a.Cin, kk = (double)cs.k * cs.k;
   const double cin_up = cs.up ? (double)cs.up->c : 0.0;   // read at a quarter of the pixels
   out.back().flops = 2.0 * (double)a.M * cout * kk * cin;
+  const double ys = a.y_f32 ? 4.0 : f8 ? (cs.y_f8 ? 1.0 : 2.0) : es, rs = f8 ? (cs.res_f8 ? 1.0 : 2.0) : es;
   out.back().bytes = (double)a.N * a.H * a.W * (cin - 0.75 * cin_up) * es + (double)cout * kk * cin * es +
-                     (double)a.M * cout * (a.y_f32 ? 4.0 : es) + (a.res ? (double)a.M * cout * es : 0.0) + 8.0 * cout;
+                     (double)a.M * cout * (ys + (a.res ? rs : 0.0)) + 8.0 * cout;
   return VRS_OK;
 }
 
@@ -531,7 +564,7 @@ static int prep_dense(vrs_ctx* ctx, const ConvSpec& spec, const vrs_nhwc& x, con
   a.M = (int32_t)M;
   a.act = cs.act;
   if (!cs.tile)
-    cs.tile = f8 ? (cout <= 64 && !cs.up ? VRS_TILE_64x256 : VRS_TILE_128x128) : auto_tile(cs, a, x, ctx->num_cu);
+    cs.tile = auto_tile(cs, a, x, ctx->num_cu);
   const size_t first = out.size();
   if ((rc = prep_tile(ctx, cs, x, cout, a, out))) return rc;
   for (size_t i = first; i < out.size(); ++i) out[i].tile = cs.tile;
@@ -1026,6 +1059,9 @@ int prep_pool(vrs_ctx* ctx, const vrs_nhwc& buf, int dtype, std::vector<Launch>&
   // cover whole 64-byte spans where the budget allows (at 3 groups, 48-byte
   // spans cost 1.8x the algorithmic HBM bytes in partial-line traffic)
   while (cg & (cg - 1)) cg &= cg - 1;
+  // fewer groups while the workgroups leave CUs idle (float32 128 channels at
+  // 20x20 x 1: 8 workgroups of two groups)
+  while (cg > 1 && (int64_t)buf.n * ((c / 8 + cg - 1) / cg) < (ctx->num_cu > 0 ? ctx->num_cu : 256)) cg /= 2;
   vrs_pool_args a{};
   a.buf = const_cast<void*>(at(buf, dtype));
   a.N = buf.n; a.H = buf.h; a.W = buf.w; a.c = c; a.pitch = buf.pitch; a.cgroups_per_block = cg;

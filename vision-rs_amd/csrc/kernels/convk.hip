@@ -3,8 +3,10 @@
 // without a workgroup while each busy one walks the whole K range.
 //
 // Semantics as conv_body.h: y = act(scale * conv(x, w) + shift) + res, folded
-// BN, bf16 or float32, any k / stride, Cin % 8 == 0, optional fused nearest-2x
-// upsample, NHWC or flat (channel-major float32) output.
+// BN, k up to 5, any stride, optional fused nearest-2x upsample, NHWC or flat
+// (channel-major float32) output; bf16 and float32 with Cin % 8 == 0, or e4m3
+// weights and activations (element type uint8_t) with Cin % 64 == 0, whose
+// output and residual are bf16 or e4m3.
 //
 // Latency bounds these layers, not bytes or flops: the time is the chain of
 // dependent waits of one workgroup.  So the output tile is one MFMA tile (32
@@ -29,6 +31,7 @@
 
 namespace {
 
+// One K slice of a TS x TS tile.
 template <typename T, int TS> struct Unit;
 template <> struct Unit<bf16_t, 32> {
   using acc_t = f32x16_t;
@@ -61,6 +64,18 @@ template <> struct Unit<float, 16> {
     for (int j = 0; j < 4; ++j)
       c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[j]), __uint_as_float(b[j]), c, 0, 0, 0);
     return c;
+  }
+};
+
+// e4m3: 32 bytes of k per lane, unit block scales
+template <> struct Unit<uint8_t, 32> {
+  using acc_t = f32x16_t;
+  static __device__ __forceinline__ acc_t mma(const i32x8_t& a, const i32x8_t& b, acc_t c) { return mfma32_fp8_k64(a, b, c); }
+};
+template <> struct Unit<uint8_t, 16> {
+  using acc_t = f32x4_t;
+  static __device__ __forceinline__ acc_t mma(const i32x8_t& a, const i32x8_t& b, acc_t c) {
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
   }
 };
 
@@ -170,7 +185,8 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
   acc_t acc;
 #pragma unroll
   for (int e = 0; e < NQ * 4; ++e) acc[e] = 0.f;
-  const int f_off = (lane % TS) * ROW + (lane / TS) * 16;
+  constexpr int FB = ES == 1 ? 32 : 16;               // bytes of a row per lane and slice
+  const int f_off = (lane % TS) * ROW + (lane / TS) * FB;
   // one step: the staged rows through this wave's own LDS (LDS operations of
   // one wave are in order: no barrier) into MFMA fragments
   auto step = [&](const u32x4_t (&wa)[RL], const u32x4_t (&wb)[RL]) {
@@ -181,14 +197,30 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
     }
   };
   auto mma = [&]() {
-    u32x4_t fa[CPS / NG], fb[CPS / NG];
+    if constexpr (ES == 1) {
+      constexpr int NS = 128 / (NG * FB);
+      i32x8_t fa[NS], fb[NS];
+      auto ld32 = [&](const unsigned char* p) {
+        const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(p), hi = *reinterpret_cast<const u32x4_t*>(p + 16);
+        return (i32x8_t){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+      };
 #pragma unroll
-    for (int s = 0; s < CPS / NG; ++s) {
-      fa[s] = *reinterpret_cast<const u32x4_t*>(sa + f_off + s * NG * 16);
-      fb[s] = *reinterpret_cast<const u32x4_t*>(sb + f_off + s * NG * 16);
+      for (int s = 0; s < NS; ++s) {
+        fa[s] = ld32(sa + f_off + s * NG * FB);
+        fb[s] = ld32(sb + f_off + s * NG * FB);
+      }
+#pragma unroll
+      for (int s = 0; s < NS; ++s) acc = Unit<T, TS>::mma(fa[s], fb[s], acc);
+    } else {
+      u32x4_t fa[CPS / NG], fb[CPS / NG];
+#pragma unroll
+      for (int s = 0; s < CPS / NG; ++s) {
+        fa[s] = *reinterpret_cast<const u32x4_t*>(sa + f_off + s * NG * 16);
+        fb[s] = *reinterpret_cast<const u32x4_t*>(sb + f_off + s * NG * 16);
+      }
+#pragma unroll
+      for (int s = 0; s < CPS / NG; ++s) acc = Unit<T, TS>::mma(fa[s], fb[s], acc);
     }
-#pragma unroll
-    for (int s = 0; s < CPS / NG; ++s) acc = Unit<T, TS>::mma(fa[s], fb[s], acc);
   };
 
 #pragma unroll
@@ -237,13 +269,18 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
       if (a.act == VRS_ACT_SILU) v[e] = silu_t<T>(v[e]);
     }
     if (a.res) {   // NHWC views: whole aligned quads (host)
-      const T* rp = reinterpret_cast<const T*>(a.res) + bb * a.r_sb + rr * a.r_sp + co;
-      if constexpr (ES == 2) {
-        const u32x2_t rv = *reinterpret_cast<const u32x2_t*>(rp);
+      const int64_t ro = bb * a.r_sb + rr * a.r_sp + co;
+      if (ES == 1 && a.res_f8) {
+        float d[4];
+        fp8x4_to_f32(*reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(a.res) + ro), a.res_step, d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += d[e];
+      } else if constexpr (ES <= 2) {
+        const u32x2_t rv = *reinterpret_cast<const u32x2_t*>(static_cast<const bf16_t*>(a.res) + ro);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] += __uint_as_float((e & 1) ? (rv[e >> 1] & 0xffff0000u) : (rv[e >> 1] << 16));
       } else {
-        const f32x4_t rv = *reinterpret_cast<const f32x4_t*>(rp);
+        const f32x4_t rv = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(a.res) + ro);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] += rv[e];
       }
@@ -254,9 +291,16 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (co + e < a.Cout) yp[e * a.y_sc] = v[e];
-    } else if constexpr (ES == 2) {
-      *reinterpret_cast<u32x2_t*>(reinterpret_cast<T*>(a.y) + yo) =
-          (u32x2_t){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    } else if constexpr (ES <= 2) {
+      const u32x2_t h = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      if (ES == 1 && a.out_step > 0.f) {   // e4m3 of the bf16 value
+        uint32_t lim = __float_as_uint(448.f * a.out_step) >> 16;
+        lim |= lim << 16;
+        *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(a.y) + yo) =
+            bf16x2_to_fp8x2(h[0], lim, a.out_step) | (bf16x2_to_fp8x2(h[1], lim, a.out_step) << 16);
+      } else {
+        *reinterpret_cast<u32x2_t*>(static_cast<bf16_t*>(a.y) + yo) = h;
+      }
     } else {
       *reinterpret_cast<f32x4_t*>(reinterpret_cast<T*>(a.y) + yo) = (f32x4_t){v[0], v[1], v[2], v[3]};
     }
@@ -310,3 +354,4 @@ constexpr int convk_waves(int ts, int kw) { return ts == 16 ? 4 : kw == 8 ? 2 : 
 // vrs_conv_<type>_s<tile>_w<waves sharing K>_<a: taps of whole steps, g: any Cin % 8 == 0>
 VRS_CONVK_TYPE(bf16, bf16_t)
 VRS_CONVK_TYPE(f32, float)
+VRS_CONVK_TYPE(fp8, uint8_t)
