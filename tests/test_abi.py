@@ -53,6 +53,29 @@ def test_null_arguments_rejected_before_any_hip_call():
     assert L.vrs_detect_workspace_size(C.byref(d)) == 0  # max_det > 1024 rejected
 
 
+def test_conv2d_reads_its_parameters_on_each_call(monkeypatch):
+    """A scale may be any object with a float value: one updated in place
+    between calls, or an unhashable one, reaches the library as it is then."""
+    import torch
+    seen = []
+
+    class Stub:
+        @staticmethod
+        def vrs_conv2d(handle, d, *rest):
+            seen.append((d._obj.in_scale, d._obj.out_step))
+            return 0
+
+    monkeypatch.setattr(vrs, "lib", lambda: Stub)
+    c = object.__new__(vrs.Context)
+    c.handle = None
+    view, t, a = vrs.Nhwc(), torch.tensor(0.5), np.array(2.0)
+    for _ in range(2):
+        c.conv2d(view, None, None, None, view, 1, in_scale=t, out_step=a, stream=0)
+        t.mul_(2)
+        a *= 2
+    assert seen == [(0.5, 2.0), (1.0, 4.0)]
+
+
 def test_pack_conv_weight_layout():
     w = np.arange(2 * 3 * 3 * 3, dtype=np.float32).reshape(2, 3, 3, 3)
     out = vrs.pack_conv_weight(w, 1, 8, vrs.F32).view(np.float32).reshape(2, 3, 3, 8)

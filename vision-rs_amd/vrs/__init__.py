@@ -14,7 +14,6 @@ psa_attention (blocks/c2psa.rs), sppf (blocks/sppf.rs), detect
 from __future__ import annotations
 
 import ctypes as C
-import functools
 import os
 
 PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -222,14 +221,6 @@ class _alloc_on:
         return False
 
 
-@functools.lru_cache(maxsize=256, typed=True)
-def _conv_desc(*fields):
-    """A ConvDesc, which the library only reads: one per distinct set of
-    parameters instead of filling twelve fields on each call (1.2 us).
-    `typed`, since a field takes an int where it refuses an equal float."""
-    return ConvDesc(*fields)
-
-
 def nhwc(t, c=None, c_off=0):
     """View of a [n, h, w, pitch] torch tensor (channels [c_off, c_off+c))."""
     n, h, w, pitch = t.shape
@@ -272,8 +263,8 @@ class Context:
         """x, y, res: Nhwc views; w/scale/shift: device tensors.  FP8: w from
         pack_conv_weight_fp8, scale including weight scale * in_scale; views of
         uint8 tensors hold e4m3 activations when x_e4m3 / y_e4m3 / res_e4m3."""
-        d = _conv_desc(k, stride, groups, act, dtype, tile, in_scale, int(x_e4m3), int(y_e4m3), int(res_e4m3),
-                       out_step, res_step)
+        d = ConvDesc(k, stride, groups, act, dtype, tile, in_scale, int(x_e4m3), int(y_e4m3), int(res_e4m3),
+                     out_step, res_step)
         check(lib().vrs_conv2d(self.handle, C.byref(d), C.byref(x), _ptr(w), _ptr(scale), _ptr(shift),
                                C.byref(res) if res is not None else None, C.byref(y), _stream(stream)))
 
