@@ -282,3 +282,33 @@ def test_split_k_fp8(n, cin, h, w, cout, k, s, res, y8, tile):
     small = (2.0 ** -9 if y8 else 1e-6) * float(a.abs().max())
     assert torch.all((a - b).abs() <= step * a.abs() + small)
     assert float((a != b).double().mean()) < 0.02   # float32 sums differ by 1e-6, roundings flip rarely
+
+
+@pytest.mark.parametrize("points", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("n,q,heads,shapes", [
+    (1, 1, 1, [(1, 1)]),                                      # one row of eight, one level, one pixel
+    (3, 7, 5, [(9, 4), (3, 1), (2, 2)]),                      # 105 rows: the last workgroup holds one
+    (2, 5, 8, [(13, 11), (7, 6), (4, 3), (2, 2)]),            # a query per workgroup
+    (1, 3, 19, [(5, 4)] * 8),                                 # eight waves, queries that straddle workgroups
+])
+def test_msda_paths(points, n, q, heads, shapes):
+    """Up to four points: a wave per level; more: the general kernel.  Points at
+    infinity and NaN, and infinite weights outside the map, add nothing."""
+    import oracle
+    import torch
+    from gpu_util import dev, rel_err
+    from test_oracle_golden import msda_inputs
+    value, ref, off, attw = msda_inputs(n, q, heads, 32, shapes, points)
+    off[0, 0, 0, 0, 0] = (np.inf, 0.0)
+    off[-1, -1, -1, -1, -1] = (np.nan, -np.inf)
+    off[0, -1, -1, 0, -1] = (50.0, 0.0)
+    clean = attw.copy()
+    for at in ((0, 0, 0, 0, 0), (-1, -1, -1, -1, -1), (0, -1, -1, 0, -1)):
+        clean[at] = 0.0
+        attw[at] = np.inf
+    exp = oracle.msda(value, shapes, ref, np.where(np.isfinite(off), off, 0).astype(np.float32), clean)
+    out = torch.full((n * q * heads * 32 + 8,), 7.0, device="cuda")
+    ctx().msda(dev(value), shapes, dev(ref), dev(off), dev(attw), out[:-8].view(n, q, heads * 32))
+    torch.cuda.synchronize()
+    assert rel_err(out[:-8].view(n, q, -1).cpu().numpy(), exp, 5e-2) < 1e-4   # the bound of the other float32 tests
+    assert torch.all(out[-8:] == 7.0)
