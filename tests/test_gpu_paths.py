@@ -312,3 +312,39 @@ def test_msda_paths(points, n, q, heads, shapes):
     torch.cuda.synchronize()
     assert rel_err(out[:-8].view(n, q, -1).cpu().numpy(), exp, 5e-2) < 1e-4   # the bound of the other float32 tests
     assert torch.all(out[-8:] == 7.0)
+
+
+@pytest.mark.parametrize("size,frames", [
+    # one canvas tile of the 2x kernel and less; a pixel; a row that no dword fits
+    (8, [(16, 16), (1, 1), (3, 1), (5, 16)]),
+    # no frame shrinks: the three-tap kernel
+    (150, [(150, 150), (61, 37), (1, 90), (149, 8)]),
+    # whole tiles; exactly 2x, 4x and 8x; one pixel more (the next kernel)
+    (64, [(128, 128), (256, 100), (512, 512), (129, 128), (257, 256), (513, 77)]),
+    # enlarged, odd row lengths, partial tiles on both sides
+    (77, [(41, 77), (77, 13), (154, 151), (301, 307), (600, 431), (77, 77)]),
+    (200, [(399, 230), (7, 200), (800, 797), (1599, 1600)]),
+])
+def test_letterbox_paths(size, frames):
+    """Frames at every byte misalignment, against the two-pass oracle bit for bit."""
+    import oracle
+    import torch
+    rng = np.random.default_rng(size)
+    offs, wh, parts, at = [], [], [], 0
+    for i in range(16):
+        w, h = frames[i % len(frames)]
+        pad = 1 + (i - 1 - at) % 16     # the frame starts at a byte = i mod 16
+        parts.append(np.full(pad, 255, np.uint8))
+        at += pad
+        offs.append(at)
+        wh.append((w, h))
+        parts.append(rng.integers(0, 256, h * w * 3, dtype=np.uint8))
+        at += h * w * 3
+    flat = np.concatenate(parts)
+    got = ctx().letterbox(torch.from_numpy(flat).cuda(), offs, wh, size)
+    torch.cuda.synchronize()
+    got = got.cpu().numpy()
+    for i, ((w, h), o) in enumerate(zip(wh, offs)):
+        assert o % 16 == i
+        ref = oracle.letterbox(flat[o:o + h * w * 3].reshape(h, w, 3), size)
+        assert np.array_equal(got[i].view(np.uint32), np.asarray(ref, np.float32).reshape(got[i].shape).view(np.uint32)), (w, h, o)

@@ -364,19 +364,22 @@ int vrs_letterbox(vrs_ctx* ctx, int32_t n, int32_t img_size, const uint8_t* rgb,
       return fail(VRS_EUNSUPPORTED, "vrs_letterbox: image %d (%dx%d) shrinks by more than 62x", i, w, h);
     ims[(size_t)i] = vrs_lb_image{off, w, h, nw, nh, (img_size - nw) / 2, (img_size - nh) / 2, i, 0};
   }
-  // per image the staged kernel for shrinks up to 2x, 4x, then
+  // per image the staged kernel for enlargements, shrinks up to 2x, 4x, then
   // VRS_LB_STAGED_RATIO x per axis (the kernels' own float32 ratio), else the
-  // direct kernel
-  auto kind = [](const vrs_lb_image& im) {
+  // direct kernel.  Enlargements go along with the 2x shrinks where a call has
+  // both: a second launch costs more than the three-tap windows save.
+  auto fits = [](const vrs_lb_image& im) {
     auto within = [&](float r) {
       return (im.nw == 0 || (float)im.w / (float)im.nw <= r) && (im.nh == 0 || (float)im.h / (float)im.nh <= r);
     };
-    return within(2.0f) ? 0 : within(4.0f) ? 1 : within((float)VRS_LB_STAGED_RATIO) ? 2 : 3;
+    return within(1.0f) ? 0 : within(2.0f) ? 1 : within(4.0f) ? 2 : within((float)VRS_LB_STAGED_RATIO) ? 3 : 4;
   };
-  static const char* names[4] = {"vrs_letterbox_f32_s2", "vrs_letterbox_f32_s4", "vrs_letterbox_f32_s8",
-                                 "vrs_letterbox_f32"};
+  const bool shrinks = std::any_of(ims.begin(), ims.end(), [&](const vrs_lb_image& im) { return fits(im) == 1; });
+  auto kind = [&](const vrs_lb_image& im) { return std::max(fits(im), shrinks ? 1 : 0); };
+  static const char* names[5] = {"vrs_letterbox_f32_s1", "vrs_letterbox_f32_s2", "vrs_letterbox_f32_s4",
+                                 "vrs_letterbox_f32_s8", "vrs_letterbox_f32"};
   std::vector<Launch> ls;
-  for (int pass = 0; pass < 4; ++pass) {
+  for (int pass = 0; pass < 5; ++pass) {
     std::vector<vrs_lb_image> sel;
     for (const auto& im : ims)
       if (kind(im) == pass) sel.push_back(im);
@@ -385,8 +388,8 @@ int vrs_letterbox(vrs_ctx* ctx, int32_t n, int32_t img_size, const uint8_t* rgb,
     hipFunction_t f;
     int rc = get_fn(ctx, name, &f);
     if (rc) return rc;
-    const int tw = pass == 2 ? 32 : 64;   // tile width; 4 rows
-    const unsigned tiles = (unsigned)(((img_size + tw - 1) / tw) * ((img_size + 3) / 4));
+    const int tw = pass == 3 ? 32 : 64, th = pass <= 1 ? 8 : 4;   // tile
+    const unsigned tiles = (unsigned)(((img_size + tw - 1) / tw) * ((img_size + th - 1) / th));
     for (size_t b0 = 0; b0 < sel.size(); b0 += VRS_LB_MAX_IMAGES) {
       vrs_lb_args a{};
       a.rgb = rgb;
@@ -395,7 +398,7 @@ int vrs_letterbox(vrs_ctx* ctx, int32_t n, int32_t img_size, const uint8_t* rgb,
       a.S = img_size;
       a.count = (int32_t)std::min<size_t>(VRS_LB_MAX_IMAGES, sel.size() - b0);
       for (int k = 0; k < a.count; ++k) a.img[k] = sel[b0 + (size_t)k];
-      ls.push_back(make_launch(name, f, dim3(tiles, (unsigned)a.count), dim3(pass == 2 ? 128 : 256), 0, a));
+      ls.push_back(make_launch(name, f, dim3(tiles, (unsigned)a.count), dim3(pass == 3 ? 128 : 256), 0, a));
     }
   }
   return run_all(ls, stream);

@@ -290,34 +290,47 @@ __device__ inline float lb_tri(float x) {
   const float a = fabsf(x);
   return a < 1.0f ? 1.0f - a : 0.0f;
 }
-// Window [lo, lo + n) of output index o along a dst-long axis from a
-// src-long one, with its normalised weights written to w[0..n) (n <= cap; the
-// host's ratio bounds keep the true window within cap).  One division per tap
-// for the weight and one for the normalisation, as the reference does them.
-__device__ inline int lb_window(int o, int src, int dst, int cap, float* w, int& lo) {
+// Window [lo, hi) of output index o along an axis of src source pixels, ratio
+// of them to an output pixel; at most `cap` taps (the host's ratio bounds keep
+// the true window within it).  c, sr: the weights' centre and support.
+__device__ inline void lb_bounds(int o, int src, float ratio, int cap, int& lo, int& hi, float& c, float& sr) {
 #pragma clang fp contract(off)
-  const float ratio = (float)src / (float)dst;
-  const float sr = ratio < 1.0f ? 1.0f : ratio;  // support 1 x sratio
+  sr = ratio < 1.0f ? 1.0f : ratio;  // support 1 x sratio
   const float centre = ((float)o + 0.5f) * ratio;
-  int l = (int)floorf(centre - sr);
-  l = l < 0 ? 0 : (l > src - 1 ? src - 1 : l);
-  int h = (int)ceilf(centre + sr);
-  h = h < l + 1 ? l + 1 : (h > src ? src : h);
-  if (h - l > cap) h = l + cap;
-  const float c = centre - 0.5f;
+  lo = (int)floorf(centre - sr);
+  lo = lo < 0 ? 0 : (lo > src - 1 ? src - 1 : lo);
+  hi = (int)ceilf(centre + sr);
+  hi = hi < lo + 1 ? lo + 1 : (hi > src ? src : hi);
+  if (hi - lo > cap) hi = lo + cap;
+  c = centre - 0.5f;
+}
+// The window of output index o with its normalised weights written to
+// w[0..n) and zeros to w[n..fill); returns n.  One division per tap for the weight and one for the
+// normalisation, as the reference does them.
+__device__ inline int lb_window(int o, int src, int dst, int cap, float* w, int& lo, int fill = 0) {
+#pragma clang fp contract(off)
+  int h;
+  float c, sr;
+  lb_bounds(o, src, (float)src / (float)dst, cap, lo, h, c, sr);
   float sum = 0.0f;
-  for (int i = l; i < h; ++i) {
+  for (int i = lo; i < h; ++i) {
     const float v = lb_tri(((float)i - c) / sr);
-    w[i - l] = v;
+    w[i - lo] = v;
     sum += v;
   }
-  for (int i = 0; i < h - l; ++i) w[i] = w[i] / sum;
-  lo = l;
-  return h - l;
+  for (int i = 0; i < h - lo; ++i) w[i] = w[i] / sum;
+  for (int i = h - lo; i < fill; ++i) w[i] = 0.0f;
+  return h - lo;
 }
-__device__ inline float lb_quant(float v) {  // clamp, round half away from zero, / 255
+// Clamp, round half away from zero, / 255.  The quotient of a whole number in
+// 0..255 by 255, correctly rounded: a product with the rounded reciprocal and
+// one residual step (Markstein), equal to the division for all 256.
+__device__ inline float lb_quant(float v) {
   v = v < 0.0f ? 0.0f : (v > 255.0f ? 255.0f : v);
-  return roundf(v) / 255.0f;
+  float q = truncf(v);
+  if (v - q >= 0.5f) q += 1.0f;
+  const float rcp = 1.0f / 255.0f, y = q * rcp;
+  return __builtin_fmaf(__builtin_fmaf(-255.0f, y, q), rcp, y);
 }
 constexpr int LB_TW = 64, LB_TH = 4, LB_LD = VRS_LB_MAX_TAPS + 1;  // odd row pitch: no bank conflicts
 }  // namespace
@@ -408,100 +421,113 @@ extern "C" __global__ __launch_bounds__(256) void vrs_letterbox_f32(vrs_lb_args 
   o[2 * plane] = lb_quant(s2);
 }
 
-// Staged variants for images shrunk at most 2x (vrs_letterbox_f32_s2), 4x
-// (_s4) or VRS_LB_STAGED_RATIO = 8x (_s8) per axis: one workgroup per 64 x 4
-// tile (32 x 4 for _s8).  After the
-// windows, the source patch the tile reads (rows spanned by its 4 row windows
-// x columns spanned by its 64 column windows) is copied into LDS with aligned
-// dword loads, all in flight together; the vertical pass then runs once per
-// (tile row, source column) from LDS into a float32 buffer, and the
-// horizontal pass reads that buffer -- the same float32 operations in the same
-// order as the direct kernel and the two-pass reference.  The patch is copied
-// in 16-byte loads so that a workgroup keeps its whole patch in flight at
-// once (the kernel is bound by loads in flight, not by bandwidth).
+// Staged variants for images enlarged or kept (vrs_letterbox_f32_s1), or shrunk
+// at most 2x (_s2), 4x (_s4) or VRS_LB_STAGED_RATIO = 8x (_s8) per axis: one
+// workgroup per TW x TH tile.  The source patch the tile reads (rows spanned by its row windows x
+// columns spanned by its column windows) is copied into LDS with aligned
+// 16-byte loads, all in flight together, while the windows' weights are
+// computed; the vertical pass then runs once per (tile row, source column)
+// from LDS into a float32 buffer, and the horizontal pass reads that buffer --
+// the same float32 operations in the same order as the direct kernel and the
+// two-pass reference.
+//
+// LDS instructions bound the vertical pass when it reads single bytes, so a
+// thread takes four pixels of a row: 12 bytes, as dwords shifted into place by
+// the row's misalignment.  Windows are padded with weights of zero to a fixed
+// length, so that a window's reads are all in flight (a sum of products >= 0
+// is unchanged by adding +0); what the padding reads is some byte of the patch
+// or a sum of them, so finite.  A window holds at most 2 R + 1 taps: its real
+// interval is 2 R long, and rounding a bound never moves it past a whole number.
+// Measured (single bytes and 4 rows a tile -> dwords and 8 rows at R <= 2): 16
+// frames of 1280 x 720 to 640 52.2 -> 40.6 us (4 rows 50.9, 16 rows 40.6, 128
+// columns 39.7), 1920 x 1080 108 -> 95, 4 of 3200 x 2160 to 640 166 -> 118.
+// VALU and LDS issue bound the small ratios (about 130 vector instructions an
+// output pixel at five taps), hence the instance of three taps (R = 1): 32
+// frames of 640 x 480 to 640 105 -> 63 us (78 on the 2x instance), 8 of 400 x
+// 300 to 1280 95.5 -> 48.6 (60.5; 3.3 TB/s).
 namespace {
 // R: the largest shrink factor per axis the instance accepts; LDS is sized
-// for it, so the small-ratio instance fits twice as many workgroups per CU
-template <int R, int LBS_TW>
+// for it, so the small-ratio instance fits more workgroups per CU
+template <int R, int TW, int TH, int NT>
 __device__ __forceinline__ void lb_staged(const vrs_lb_args& a) {
 #pragma clang fp contract(off)
-  constexpr int LBS_TH = 4, NT = LBS_TW * LBS_TH, LBS_TAPS = 2 * R + 2, LBS_LD = LBS_TAPS + 1;
+  constexpr int TAPS = 2 * R + 1, U = R == 2 ? 5 : R <= 4 ? 3 : 6;   // taps in flight
+  constexpr int PAD = (TAPS + U - 1) / U * U;                          // padded window
+  // weights: a window per thread, or, of more taps, a tap (17 taps: 34 divisions
+  // in a row, 338 us for 16 frames of 3100 x 2400 to 416; by tap 295, but 41.5
+  // instead of 40.9 at 5 taps)
+  constexpr bool BY_TAP = R > 4;
+  constexpr int LDC = PAD | 1, LDR = (PAD + 3) / 4 * 4;
   // source columns / rows a tile touches: (n - 1) * ratio + 2 * ratio + 2, +2 slack
-  constexpr int LBS_CMAX = (LBS_TW - 1) * R + 2 * R + 4;
-  constexpr int LBS_RMAX = (LBS_TH - 1) * R + 2 * R + 4;
-  constexpr int LBS_PW = (LBS_CMAX * 3 + 15 + 15) / 16;   // 16-byte chunks per patch row (15-byte lead-in)
-  constexpr int LBS_VREG = 4;                               // chunks in flight per thread and round
-  __shared__ float wcol[LBS_TW * LBS_LD];
-  __shared__ float wrow[LBS_TH * LBS_LD];
-  __shared__ int gcol[LBS_TW][2], grow[LBS_TH][2];
-  __shared__ u32x4_t patch[LBS_RMAX * LBS_PW];
-  __shared__ int plead[LBS_RMAX];
-  __shared__ float vbuf[LBS_TH * LBS_CMAX * 3];
+  constexpr int CMAX = (TW - 1) * R + 2 * R + 4;
+  constexpr int RMAX = (TH - 1) * R + 2 * R + 4;
+  constexpr int VU = (CMAX + U + 3) / 4;               // units of 4 pixels, the padding's reads included
+  constexpr int PW = (15 + 12 * VU + 4 + 15) / 16;     // 16-byte chunks per patch row (15-byte lead-in)
+  constexpr int CL = PW <= 32 ? 32 : 64;               // lanes that copy one row
+  constexpr int RPR = NT / CL, ROUNDS = (RMAX + RPR - 1) / RPR, VREG = ROUNDS < 4 ? ROUNDS : 4;
+  static_assert(PW <= 64 && TW + TH <= NT && NT % TW == 0, "tile");
+  __shared__ float wcol[TW * LDC];
+  __shared__ __attribute__((aligned(16))) float wrow[TH * LDR];
+  __shared__ int gcol[TW][2], grow[TH][2];
+  __shared__ u32x4_t patch[RMAX * PW];
+  __shared__ __attribute__((aligned(16))) float vbuf[TH * VU * 12];
+  float* const raw = vbuf;                             // the unnormalised weights, before the vertical pass
+  static_assert((TW + TH) * PAD <= TH * VU * 12, "weights fit");
   const vrs_lb_image im = a.img[blockIdx.y];
-  const int tiles_x = (a.S + LBS_TW - 1) / LBS_TW;
-  const int x0 = (int)(blockIdx.x % tiles_x) * LBS_TW, y0 = (int)(blockIdx.x / tiles_x) * LBS_TH;
+  const int tiles_x = (a.S + TW - 1) / TW;
+  const int x0 = (int)(blockIdx.x % tiles_x) * TW, y0 = (int)(blockIdx.x / tiles_x) * TH;
   const int64_t plane = (int64_t)a.S * a.S;
   float* ob = a.out + (int64_t)im.slot * 3 * plane;
   const int t = threadIdx.x;
-  const int tx = t % LBS_TW, ty = t / LBS_TW;
-  const int ox = x0 + tx, oy = y0 + ty;
+  const int tx = t % TW, ty = t / TW;
+  const int ox = x0 + tx;
   // in-image columns [cf, cl] and rows [rf, rl] of the tile (uniform)
-  const int cf = max(im.px - x0, 0), cl = min(im.px + im.nw - x0, LBS_TW) - 1;
-  const int rf = max(im.py - y0, 0), rl = min(im.py + im.nh - y0, LBS_TH) - 1;
+  const int cf = max(im.px - x0, 0), cl = min(im.px + im.nw - x0, TW) - 1;
+  const int rf = max(im.py - y0, 0), rl = min(im.py + im.nh - y0, TH) - 1;
   if (cf > cl || rf > rl) {   // all padding
-    if (ox < a.S && oy < a.S) {
-      float* o = ob + (int64_t)oy * a.S + ox;
+    for (int r = ty; r < TH; r += NT / TW) {
+      if (ox >= a.S || y0 + r >= a.S) continue;
+      float* o = ob + (int64_t)(y0 + r) * a.S + ox;
       o[0] = a.pad;
       o[plane] = a.pad;
       o[2 * plane] = a.pad;
     }
     return;
   }
-  if (t < LBS_TW) {
-    if (t >= cf && t <= cl) {
-      int lo;
-      const int n = lb_window(x0 + t - im.px, im.w, im.nw, LBS_TAPS, wcol + t * LBS_LD, lo);
-      gcol[t][0] = lo;
-      gcol[t][1] = lo + n;
-    }
-  } else if (t < LBS_TW + LBS_TH) {
-    const int r = t - LBS_TW;
-    if (r >= rf && r <= rl) {
-      int lo;
-      const int n = lb_window(y0 + r - im.py, im.h, im.nh, LBS_TAPS, wrow + r * LBS_LD, lo);
-      grow[r][0] = lo;
-      grow[r][1] = lo + n;
-    }
-  }
-  __syncthreads();
   // window bounds are non-decreasing along an axis: the patch is source rows
   // [top of the first row window, bottom of the last) x columns [lo of the
   // first column window, hi of the last)
-  const int c_lo = gcol[cf][0];
-  const int ncol = min(gcol[cl][1] - c_lo, LBS_CMAX);   // <= LBS_CMAX and LBS_RMAX by the ratio bound
-  const int ytop = grow[rf][0];
-  const int nrow = min(grow[rl][1] - ytop, LBS_RMAX);
+  int c_lo, ytop, hi, skip;
+  float f0, f1;
+  const float ratio_x = (float)im.w / (float)im.nw, ratio_y = (float)im.h / (float)im.nh;
+  lb_bounds(x0 + cf - im.px, im.w, ratio_x, TAPS, c_lo, skip, f0, f1);
+  lb_bounds(x0 + cl - im.px, im.w, ratio_x, TAPS, skip, hi, f0, f1);
+  const int ncol = min(hi - c_lo, CMAX);   // <= CMAX and RMAX by the ratio bound
+  lb_bounds(y0 + rf - im.py, im.h, ratio_y, TAPS, ytop, skip, f0, f1);
+  lb_bounds(y0 + rl - im.py, im.h, ratio_y, TAPS, skip, hi, f0, f1);
+  const int nrow = min(hi - ytop, RMAX);
   // patch row i holds the source bytes [s_i, s_i + 3*ncol) of image row
   // ytop + i (s_i = off + ((ytop + i)*w + c_lo)*3), copied as the 16-byte
-  // aligned chunks that cover them; the bytes start at plead[i] = address of
-  // s_i mod 16.  Chunks straddling the image's first or last byte (only
-  // those) are assembled from byte loads.
+  // aligned chunks that cover them, so its bytes start at s_i's address mod
+  // 16.  Chunks straddling the image's first or last byte (only those) are
+  // assembled from byte loads.
   const unsigned char* img0 = a.rgb + im.off;
   const unsigned char* img1 = img0 + (int64_t)im.w * im.h * 3;
-  const int nq = (3 * ncol + 15 + 15) / 16;   // chunks per row copy (<= LBS_PW)
-  const int total = nrow * nq;
-  if (t < nrow)
-    plead[t] = (int)(reinterpret_cast<uintptr_t>(img0 + ((int64_t)(ytop + t) * im.w + c_lo) * 3) & 15);
-  for (int base = t; base < total; base += NT * LBS_VREG) {
-    u32x4_t v[LBS_VREG];
+  const unsigned char* src = img0 + ((int64_t)ytop * im.w + c_lo) * 3;
+  const int64_t stride = (int64_t)im.w * 3;
+  const uint32_t lead0 = (uint32_t)(reinterpret_cast<uintptr_t>(src) & 15), dlead = (uint32_t)stride;
+  const int nq = (3 * ncol + 15 + 15) / 16;   // chunks per row copy (<= PW)
+  const int cd = t % CL, cr = t / CL;
+#pragma unroll 1
+  for (int base = 0; base < ROUNDS; base += VREG) {
+    u32x4_t v[VREG];
 #pragma unroll
-    for (int u = 0; u < LBS_VREG; ++u) {
-      const int idx = base + u * NT;
-      if (idx < total) {
-        const int i = idx / nq, d = idx - (idx / nq) * nq;
-        const unsigned char* row_p = img0 + ((int64_t)(ytop + i) * im.w + c_lo) * 3;
+    for (int u = 0; u < VREG; ++u) {
+      const int i = cr + (base + u) * RPR;
+      v[u] = (u32x4_t){0, 0, 0, 0};
+      if (i < nrow && cd < nq) {
         const unsigned char* q = reinterpret_cast<const unsigned char*>(
-            (reinterpret_cast<uintptr_t>(row_p) & ~(uintptr_t)15) + 16 * (uintptr_t)d);
+            (reinterpret_cast<uintptr_t>(src + i * stride) & ~(uintptr_t)15) + 16 * (uintptr_t)cd);
         if (q >= img0 && q + 16 <= img1) {
           v[u] = *reinterpret_cast<const u32x4_t*>(q);
         } else {
@@ -512,66 +538,143 @@ __device__ __forceinline__ void lb_staged(const vrs_lb_args& a) {
         }
       }
     }
+    if (base == 0) {   // the windows, under the first loads
+      if constexpr (BY_TAP) {   // a tap per thread, zero past a window's end
+        for (int k = t; k < (TW + TH) * PAD; k += NT) {
+          const int g = k / PAD, i = k - g * PAD;
+          const bool col = g < TW;
+          const int p = col ? x0 + g - im.px : y0 + g - TW - im.py;
+          float v = 0.0f;
+          if (p >= 0 && p < (col ? im.nw : im.nh)) {
+            int lo, h;
+            float c, sr;
+            lb_bounds(p, col ? im.w : im.h, col ? ratio_x : ratio_y, TAPS, lo, h, c, sr);
+            if (i < h - lo) v = lb_tri(((float)(lo + i) - c) / sr);
+            if (i == 0) {
+              int* e = col ? gcol[g] : grow[g - TW];
+              e[0] = lo - (col ? c_lo : ytop);
+              e[1] = h - lo;
+            }
+          }
+          raw[k] = v;
+        }
+        __syncthreads();
+        for (int k = t; k < (TW + TH) * PAD; k += NT) {
+          const int g = k / PAD, i = k - g * PAD;
+          float sum = 0.0f;
 #pragma unroll
-    for (int u = 0; u < LBS_VREG; ++u) {
-      const int idx = base + u * NT;
-      if (idx < total) patch[(idx / nq) * LBS_PW + idx % nq] = v[u];
-    }
-  }
-  __syncthreads();
-  // vertical pass: one (tile row, patch column) per thread and step; the row
-  // loop is uniform over the workgroup
-  const unsigned char* pb = reinterpret_cast<const unsigned char*>(patch);
-  for (int r = rf; r <= rl; ++r) {
-    const int top = grow[r][0], n = grow[r][1] - top;
-    const float* wy = wrow + r * LBS_LD;
-    for (int x = t; x < ncol; x += NT) {
-      float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
-      for (int j = 0; j < n; ++j) {
-        const int i = top - ytop + j;
-        const unsigned char* q = pb + i * LBS_PW * 16 + plead[i] + x * 3;
-        const float w = wy[j];
-        t0 += (float)q[0] * w;
-        t1 += (float)q[1] * w;
-        t2 += (float)q[2] * w;
+          for (int e = 0; e < PAD; ++e) sum += raw[g * PAD + e];
+          (g < TW ? wcol + g * LDC : wrow + (g - TW) * LDR)[i] = raw[k] / sum;
+        }
+      } else if (t < TW) {
+        if (t >= cf && t <= cl) {
+          int lo;
+          gcol[t][1] = lb_window(x0 + t - im.px, im.w, im.nw, TAPS, wcol + t * LDC, lo, PAD);
+          gcol[t][0] = lo - c_lo;
+        }
+      } else if (t < TW + TH) {
+        const int r = t - TW;
+        if (r >= rf && r <= rl) {
+          int lo;
+          grow[r][1] = lb_window(y0 + r - im.py, im.h, im.nh, TAPS, wrow + r * LDR, lo, PAD);
+          grow[r][0] = lo - ytop;
+        }
       }
-      float* vv = vbuf + (r * LBS_CMAX + x) * 3;
-      vv[0] = t0;
-      vv[1] = t1;
-      vv[2] = t2;
+    }
+#pragma unroll
+    for (int u = 0; u < VREG; ++u) {
+      const int i = cr + (base + u) * RPR;
+      if (i < nrow && cd < nq) patch[i * PW + cd] = v[u];
     }
   }
   __syncthreads();
-  // horizontal pass, one pixel per thread
-  if (ox >= a.S || oy >= a.S) return;
-  float* o = ob + (int64_t)oy * a.S + ox;
-  if (tx < cf || tx > cl || ty < rf || ty > rl) {
-    o[0] = a.pad;
-    o[plane] = a.pad;
-    o[2 * plane] = a.pad;
-    return;
+  // vertical pass: one unit of four source columns of a tile row per thread
+  // and step, the columns that the horizontal padding reads included
+  const uint32_t* pd = reinterpret_cast<const uint32_t*>(patch);
+  const int nu = min((ncol + U + 3) / 4, VU);
+  const int units = (rl - rf + 1) * nu;
+  const float inv_nu = 1.0f / (float)nu;
+  for (int idx = t; idx < units; idx += NT) {
+    int u;
+    const int r = rf + fdivmod(idx, nu, inv_nu, u);
+    const int top = grow[r][0], n = grow[r][1];
+    const float* wy = wrow + r * LDR;
+    float acc[12];
+#pragma unroll
+    for (int e = 0; e < 12; ++e) acc[e] = 0.0f;
+#pragma unroll
+    for (int j0 = 0; j0 < PAD; j0 += U) {
+      if (j0 >= n) break;
+      uint32_t q[U][4], sh[U];
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const int i = min(top + j0 + j, nrow - 1);
+        const uint32_t lead = (lead0 + (uint32_t)i * dlead) & 15;
+        const uint32_t* p = pd + i * (PW * 4) + (lead >> 2) + 3 * u;
+        sh[j] = lead & 3;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[j][e] = p[e];
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const float w = wy[j0 + j];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          const uint32_t d = __builtin_amdgcn_alignbyte(q[j][e + 1], q[j][e], sh[j]);
+          acc[4 * e + 0] += (float)(d & 0xff) * w;
+          acc[4 * e + 1] += (float)(d >> 8 & 0xff) * w;
+          acc[4 * e + 2] += (float)(d >> 16 & 0xff) * w;
+          acc[4 * e + 3] += (float)(d >> 24) * w;
+        }
+      }
+    }
+    f32x4_t* vv = reinterpret_cast<f32x4_t*>(vbuf + (r * VU + u) * 12);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) vv[e] = (f32x4_t){acc[4 * e], acc[4 * e + 1], acc[4 * e + 2], acc[4 * e + 3]};
   }
-  const int lo = gcol[tx][0], n = min(gcol[tx][1], c_lo + ncol) - lo;
-  const float* vv = vbuf + (ty * LBS_CMAX + lo - c_lo) * 3;
-  const float* wx = wcol + tx * LBS_LD;
-  float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-  for (int i = 0; i < n; ++i) {
-    const float w = wx[i];
-    s0 += vv[3 * i] * w;
-    s1 += vv[3 * i + 1] * w;
-    s2 += vv[3 * i + 2] * w;
+  __syncthreads();
+  // horizontal pass: a column per thread, its weights held over the rows
+  if (ox >= a.S) return;
+  const bool in_x = tx >= cf && tx <= cl;
+  const int lo = in_x ? gcol[tx][0] : 0, n = in_x ? min(gcol[tx][1], ncol - lo) : 0;
+#pragma unroll
+  for (int r0 = 0; r0 < TH; r0 += NT / TW) {
+    const int r = r0 + ty;
+    if (y0 + r >= a.S) continue;
+    float* o = ob + (int64_t)(y0 + r) * a.S + ox;
+    if (!in_x || r < rf || r > rl) {
+      o[0] = a.pad;
+      o[plane] = a.pad;
+      o[2 * plane] = a.pad;
+      continue;
+    }
+    const float* vv = vbuf + r * (VU * 12) + lo * 3;
+    const float* wx = wcol + tx * LDC;
+    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+    for (int i0 = 0; i0 < PAD; i0 += U) {
+      if (i0 >= n) break;
+#pragma unroll
+      for (int i = i0; i < i0 + U; ++i) {
+        const float w = wx[i];
+        s0 += vv[3 * i] * w;
+        s1 += vv[3 * i + 1] * w;
+        s2 += vv[3 * i + 2] * w;
+      }
+    }
+    o[0] = lb_quant(s0);
+    o[plane] = lb_quant(s1);
+    o[2 * plane] = lb_quant(s2);
   }
-  o[0] = lb_quant(s0);
-  o[plane] = lb_quant(s1);
-  o[2 * plane] = lb_quant(s2);
 }
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(256) void vrs_letterbox_f32_s2(vrs_lb_args a) { lb_staged<2, 64>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_letterbox_f32_s4(vrs_lb_args a) { lb_staged<4, 64>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_letterbox_f32_s1(vrs_lb_args a) { lb_staged<1, 64, 8, 256>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_letterbox_f32_s2(vrs_lb_args a) { lb_staged<2, 64, 8, 256>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_letterbox_f32_s4(vrs_lb_args a) { lb_staged<4, 64, 4, 256>(a); }
 // 32 x 4 tiles (128 threads) keep the patch of an 8x shrink within 40 KB of LDS
 extern "C" __global__ __launch_bounds__(128) void vrs_letterbox_f32_s8(vrs_lb_args a) {
-  lb_staged<VRS_LB_STAGED_RATIO, 32>(a);
+  lb_staged<VRS_LB_STAGED_RATIO, 32, 4, 128>(a);
 }
 
 // Grid-unit decode on [B,4,A] rows l,t,r,b (kernels/detect_decode.rs:36-86):
