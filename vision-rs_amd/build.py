@@ -25,8 +25,8 @@ LIB = os.path.join(PKG, "lib")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-# Packed-FP32 VALU forms are disabled for every device compile (their results
-# have been unreliable on this pool); -O3 would otherwise emit them.
+# Packed-FP32 VALU forms are disabled for every device compile (some of their forms
+# have given wrong results on MI355X); -O3 would otherwise emit them.
 DEVICE_FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}",
                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-result",
