@@ -814,12 +814,12 @@ static int prep_grouped(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, con
 // Output tile of the LDS-tile depthwise kernel (tile_h x tile_w and the tile
 // counts of `a`); returns the workgroups.  Least predicted time: the latency
 // of one workgroup (t[0] + t[1] per round of 512 input pixels + t[2] per round
-// of 64 strips) plus, for each further workgroup per CU, its share of loads
-// (t[3]), strips (t[4]) and start (t[5]); microseconds, fitted to 17 shapes x
-// up to 30 tiles per kernel (rms error 8-10 %; the tile it picks is 2-4 % over
-// the best).
+// of 256 strip parts of four channels) plus, for each further workgroup per CU, its share of loads
+// (t[3]), strips (t[4]) and start (t[5]); microseconds, fitted to 14-17
+// shapes x up to 30 tiles per kernel (rms error 8-10 %; the tile it picks is
+// 1-4 % over the best).
 static int64_t dw_tile(int dtype, int stride, int n, int c, int ho, int wo, int num_cu, vrs_dw_args& a) {
-  static const double kBf16[6] = {2.57, 1.11, 1.92, 0.894, 0.638, 1.19}, kF32[6] = {2.26, 1.10, 1.90, 1.76, 0.294, 0.421},
+  static const double kBf16[6] = {2.25, 0.708, 1.47, 1.86, 0, 0.504}, kF32[6] = {2.26, 1.10, 1.90, 1.76, 0.294, 0.421},
                       kF32s2[6] = {3.01, 1.32, 0.893, 1.14, 0.037, 0.477};
   const double* t = dtype == VRS_BF16 ? kBf16 : stride == 1 ? kF32 : kF32s2;
   // (float32 stride 1: three workgroups share a CU's LDS up to 44 KB)
@@ -833,7 +833,8 @@ static int64_t dw_tile(int dtype, int stride, int n, int c, int ho, int wo, int 
       const int px = ((th - 1) * stride + 3) * ((tw - 1) * stride + 3);
       if (px * 64 > cap) continue;
       const int64_t wg = n * blocks * ((ho + th - 1) / th) * ((wo + tw - 1) / tw);
-      const double strips = ((th + 3) / 4 * tw + 63) / 64;
+      const int round = dtype == VRS_BF16 ? 32 : 64;   // strips: a thread takes four channels of 64 bytes
+      const double strips = ((th + 3) / 4 * tw + round - 1) / round;
       const double us = t[0] + t[1] * ((px + 511) / 512) + t[2] * strips +
                         std::max(0.0, (double)wg / (num_cu > 0 ? num_cu : 256) - 1.0) *
                             (t[3] * px / 512 + t[4] * strips + t[5]);

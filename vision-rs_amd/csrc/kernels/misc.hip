@@ -257,19 +257,23 @@ extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s2_bf16(vrs_dw_arg
 // bytes of channels (4 chunks of 16 bytes) of a tile_h x tile_w output tile:
 // all its input chunks are requested at once (eight in flight per thread),
 // written to LDS, and each thread computes strips of DT_R output rows of one
-// column from there, so the time is one memory latency plus the arithmetic.
+// column and four channels from there, so the time is one memory latency plus
+// the arithmetic.
 // Sums in the walker's order: the same bits.  Measured, walker -> tile:
 // float32 64 channels at 80x80 x 1 38.6 -> 5.2 us, 256 at 80x80 x 32 (419 MB)
 // 117 -> 109 us; stride 2 (one thread per output strip before) 512 at 40x40 x 1
 // 8.5 -> 5.4 us, 256 at 80x80 x 32 77 -> 58 us; bfloat16 64 at 80x80 x 1 22.5 ->
-// 5.2 us, 256 at 80x80 x 4 24.3 -> 12.4 us, 512 at 20x20 x 32 12.5 -> 11.4 us
-// (a copy of it 7.5), 256 at 80x80 x 32 52 -> 57 us (walker kept).
+// 4.4 us, 256 at 80x80 x 4 24.3 -> 11.1 us, 512 at 20x20 x 32 12.5 -> 10.8 us
+// (a copy of it 7.5), 256 at 80x80 x 32 52 -> 57 us (walker kept).  Four
+// channels a thread also in bfloat16: with eight, the 72 float weights left two
+// waves per SIMD (11.4 us at 20x20 x 32, 4.9 at 80x80 x 1, 9.8 for 304 channels
+// at 13x11 x 64, now 7.8).
 namespace {
 constexpr int DT_R = 4;   // output rows per thread and strip
 
 template <typename T, int S>
 __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
-  constexpr int EPC = 16 / (int)sizeof(T);       // channels per chunk
+  constexpr int EPC = 4, CB = EPC * (int)sizeof(T), LPP = 64 / CB;   // channels and bytes per thread, threads per pixel
   constexpr int NR = (DT_R - 1) * S + 3;         // input rows of a strip
   extern __shared__ __attribute__((aligned(16))) unsigned char dwt_lds[];
   u32x4_t* tile = reinterpret_cast<u32x4_t*>(dwt_lds);   // [input row][input column][chunk]
@@ -283,15 +287,16 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
   const int ic = (a.tile_w - 1) * S + 3;
   const int rows = min(a.tile_h, a.Ho - oy0), cols = min(a.tile_w, a.Wo - ox0);
   const int ir = (rows - 1) * S + 3;
-  const int ch = tid & 3;
-  const int c0 = cb * 4 * EPC + ch * EPC;
+  const int ch = tid % LPP;
+  const int c0 = cb * (64 / (int)sizeof(T)) + ch * EPC;
   const bool cok = c0 < a.C;
 
-  // this thread's weights and constants (its chunk is the same for every item)
-  u32x4_t wq[9];
+  // this thread's weights and constants (its channels are the same for every item)
+  typedef uint32_t part_t __attribute__((ext_vector_type(CB / 4)));
+  part_t wq[9];
   const T* wp = reinterpret_cast<const T*>(a.w) + (cok ? c0 : 0);
 #pragma unroll
-  for (int k = 0; k < 9; ++k) wq[k] = *reinterpret_cast<const u32x4_t*>(wp + (int64_t)k * a.C);
+  for (int k = 0; k < 9; ++k) wq[k] = *reinterpret_cast<const part_t*>(wp + (int64_t)k * a.C);
   float sc[EPC], sh[EPC];
 #pragma unroll
   for (int e = 0; e < EPC; ++e) {
@@ -299,7 +304,10 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
     sh[e] = a.shift[(cok ? c0 : 0) + e];
   }
 
-  const T* x = reinterpret_cast<const T*>(a.x) + (int64_t)b * a.H * a.W * a.x_pitch + c0;
+  // staging: 16-byte chunks, four threads a pixel
+  const int sch = tid & 3, sc0 = cb * (64 / (int)sizeof(T)) + sch * (16 / (int)sizeof(T));
+  const bool sok = sc0 < a.C;
+  const T* x = reinterpret_cast<const T*>(a.x) + (int64_t)b * a.H * a.W * a.x_pitch + sc0;
   const int iy0 = oy0 * S - 1, ix0 = ox0 * S - 1;
   const float inv_ic = 1.0f / (float)ic;
   const int npx = ir * ic;
@@ -313,20 +321,20 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
       const int ry = fdivmod(min(p, npx - 1), ic, inv_ic, cx);
       const int iy = iy0 + ry, ix = ix0 + cx;
       v[i] = (u32x4_t){0, 0, 0, 0};
-      if (p < npx && cok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W)
+      if (p < npx && sok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W)
         v[i] = *reinterpret_cast<const u32x4_t*>(x + ((int64_t)iy * a.W + ix) * a.x_pitch);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i)
-      if (p0 + i * 64 < npx) tile[(p0 + i * 64) * 4 + ch] = v[i];
+      if (p0 + i * 64 < npx) tile[(p0 + i * 64) * 4 + sch] = v[i];
   }
   __syncthreads();
   if (!cok) return;
 
-  auto chunk = [&](const u32x4_t& q, float (&o)[EPC]) {
+  auto chunk = [&](const part_t& q, float (&o)[EPC]) {
     if constexpr (sizeof(T) == 2) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
+      for (int e = 0; e < 2; ++e) {
         o[2 * e] = __uint_as_float(q[e] << 16);
         o[2 * e + 1] = __uint_as_float(q[e] & 0xffff0000u);
       }
@@ -341,7 +349,7 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
   T* y = reinterpret_cast<T*>(a.y);
   const int strips = (rows + DT_R - 1) / DT_R, items = strips * cols;
   const float inv_cols = 1.0f / (float)cols;
-  for (int it = tid >> 2; it < items; it += 64) {
+  for (int it = tid / LPP; it < items; it += 256 / LPP) {
     int ox;
     const int st = fdivmod(it, cols, inv_cols, ox);
     float acc[DT_R][EPC];
@@ -354,11 +362,11 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
 #pragma unroll
     for (int rr = 0; rr < NR; ++rr) {
       const int row = min(st * DT_R * S + rr, ir - 1);
-      const u32x4_t* t = tile + (row * ic + ox * S) * 4 + ch;
+      const part_t* t = reinterpret_cast<const part_t*>(tile) + (row * ic + ox * S) * LPP + ch;
 #pragma unroll
       for (int kx = 0; kx < 3; ++kx) {
         float xv[EPC];
-        chunk(t[kx * 4], xv);
+        chunk(t[kx * LPP], xv);
 #pragma unroll
         for (int r = 0; r < DT_R; ++r) {
           const int ky = rr - r * S;
@@ -377,19 +385,17 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
         v[e] = acc[r][e] * sc[e] + sh[e];
         if (a.act == VRS_ACT_SILU) v[e] = silu_t<T>(v[e]);
       }
-      u32x4_t o;
+      part_t o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+      for (int e = 0; e < CB / 4; ++e)
         o[e] = sizeof(T) == 2 ? pack_bf16x2(v[(2 * e) % EPC], v[(2 * e + 1) % EPC]) : __float_as_uint(v[e]);
-      *reinterpret_cast<u32x4_t*>(y + (((int64_t)b * a.Ho + oy0 + st * DT_R + r) * a.Wo + ox0 + ox) * a.y_pitch + c0) = o;
+      *reinterpret_cast<part_t*>(y + (((int64_t)b * a.Ho + oy0 + st * DT_R + r) * a.Wo + ox0 + ox) * a.y_pitch + c0) = o;
     }
   }
 }
 }  // namespace
 
-// (bfloat16: 72 float weights and 8-channel strips take 180 registers; three
-// waves per SIMD spilled, 6.6 against 5.2 us on the smallest problems)
-extern "C" __global__ __launch_bounds__(256, 2) void vrs_dwconv3_t1_bf16(vrs_dw_args a) { dwt_body<bf16_t, 1>(a); }
+extern "C" __global__ __launch_bounds__(256, 4) void vrs_dwconv3_t1_bf16(vrs_dw_args a) { dwt_body<bf16_t, 1>(a); }
 extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_t1_f32(vrs_dw_args a) { dwt_body<float, 1>(a); }
 extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_t2_f32(vrs_dw_args a) { dwt_body<float, 2>(a); }
 
