@@ -98,6 +98,34 @@ def test_fp8_forced_mode_keeps_every_eligible_conv_on_fp8():
             assert not ios[i].y_e4m3, pre
 
 
+@pytest.mark.parametrize("variant,batch,size,mode", [("n", 1, 128, 1), ("m", 1, 320, 1), ("m", 2, 256, 1), ("m", 1, 128, 2)])
+def test_autotuned_fp8_model_of_small_maps(variant, batch, size, mode):
+    """Small maps, where an fp8 conv's automatic tile is a split-K one (e4m3
+    input only) and bf16 and fp8 layers mix: no conv keeps such a tile on a
+    bfloat16 input, the model runs, and its plan applied to a fresh model
+    gives the same plan and bits."""
+    import torch
+    x = dev(np.random.default_rng(8).uniform(0, 1, (batch, 3, size, size)).astype(np.float32))
+    desc = vrs.block(vrs.BLOCK_YOLO26, 3, nc=80, variant=variant, one2one=True)
+    outs, plan = [], None
+    for _ in range(2):
+        m = vrs.Model(ctx(), desc, batch, size, size, vrs.FP8, 1e-3, autotune=mode)
+        if plan is not None:
+            m.set_plan(plan)
+        m.load(_params(m))
+        m.calibrate(x)
+        assert plan is None or m.get_plan() == plan
+        plan = m.get_plan()
+        outs.append([o.clone() for o in m.forward(x)])
+        torch.cuda.synchronize()
+        split = lambda p: p & 0xff in (vrs.TILE_KW16, vrs.TILE_KW32)
+        ios = [m.conv_io(i) for i in range(len(plan))]
+        assert any(io.fp8 and not io.x_e4m3 for io in ios)
+        assert not any(io.fp8 and not io.x_e4m3 and split(p) for io, p in zip(ios, plan))
+    for a, b in zip(*outs):
+        assert torch.isfinite(a).all() and torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 def test_conv_io_views():
     """conv_io describes each conv: launch order, views inside the model's
     buffers, the stem and the flat Detect outputs."""

@@ -1517,12 +1517,14 @@ int vrs_model_finalize(vrs_model* m) {
   if (!rc) plan_e4m3(m);
   // The storage is final only now: the tiles were timed on the storage of an
   // all-fp8 model, and a buffer whose reader or writer then chose bfloat16
-  // stays bfloat16, so an fp8 conv reading it drops what needs an e4m3 input
-  // (128-deep steps; the 64-deep tile takes either input).
+  // stays bfloat16, so an fp8 conv reading it drops what needs an e4m3 input:
+  // 128-deep steps (the 64-deep tile takes either input) and the split-K tiles
+  // (the automatic choice for a bfloat16 input instead).
   if (!rc && m->plan.empty())
-    for (ConvStep& c : m->convs)
-      if (c.f8 && c.run_f8 && (c.tile8 & VRS_TILE_K128) && !(c.x.buf >= 0 && m->bufs[c.x.buf].f8))
-        c.tile8 &= ~VRS_TILE_K128;
+    for (ConvStep& c : m->convs) {
+      if (!c.f8 || !c.run_f8 || (c.x.buf >= 0 && m->bufs[c.x.buf].f8)) continue;
+      c.tile8 = split_k_tile(c.tile8) ? VRS_TILE_AUTO : c.tile8 & ~VRS_TILE_K128;
+    }
   if (rc) {
     const std::string err = vrs_last_error();
     for (size_t i = first_alloc; i < m->allocs.size(); ++i) (void)hipFree(m->allocs[i]);
