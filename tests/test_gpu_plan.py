@@ -335,6 +335,29 @@ def test_head_outputs_on_the_weight_stationary_tile():
         assert torch.equal(a.view(torch.int32), b.view(torch.int32))
 
 
+def test_unaligned_outputs_keep_the_bits_of_the_weight_stationary_tile():
+    """Head outputs planned on the weight-stationary tile, of maps small enough
+    that the automatic tile is a split-K one: output tensors off 16 bytes run on
+    the tiled kernels, with the bits of the aligned call."""
+    import torch
+    x = dev(np.random.default_rng(13).uniform(0, 1, (1, 3, 128, 128)).astype(np.float32))
+    m = _yolo(1, 128, vrs.BF16, autotune=False)
+    heads = [i for i, (p, _, _) in enumerate(m.conv_info()) if p.startswith("model.23.") and p.endswith(".2")]
+    m.set_plan([vrs.TILE_W1_128 if i in heads else 0 for i in range(len(m.conv_info()))])
+    m.load(_params(m))
+    outs = []
+    for off in (0, 1):
+        flat = [torch.zeros(o.numel() + 4, device="cuda") for o in m.alloc_outputs()]
+        outs.append([t[off:off + t.numel() - 4] for t in flat])
+        m.forward(x, outs[-1])
+        names = m.launch_names()
+        on_w1 = [names[m.conv_io(i).launch].endswith("_f") for i in heads]
+        assert all(on_w1) if off == 0 else not any(on_w1), names
+    torch.cuda.synchronize()
+    for a, b in zip(*outs):
+        assert a.any() and torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 def test_fused_upsample_on_the_256x256_tile():
     """The neck's fused-upsample 1x1 convs (model.13.cv1, model.16.cv1) on the
     256x256 tile, and model.16.cv1's leftover pixel tiles on the 128x128

@@ -947,11 +947,12 @@ int prepare(vrs_model* m, const float* x, float* const* outs) {
                               c.sb, c.sp, c.sc, ls);
           // the weight-stationary float32-output tile stores 16-byte pixel
           // quads, so it needs a 16-byte aligned output slice; on a caller's
-          // output that is not, the conv runs on the tiled kernel instead
-          // (same results: the same K order per output)
+          // output that is not, the conv runs on a tiled kernel instead (same
+          // results: the same K order per output, which the automatic tile,
+          // a split-K one for small maps, would not keep)
           if (rc == VRS_EUNSUPPORTED && ((cs.tile & 0xff) == VRS_TILE_W1_128 || (cs.tile & 0xff) == VRS_TILE_W1_256)) {
             ls.resize(conv_first);
-            cs.tile = VRS_TILE_AUTO;
+            cs.tile = c.cout <= 64 ? VRS_TILE_64x256 : VRS_TILE_128x128;
             rc = prep_conv_flat(m->ctx, cs, view_of(m, c.x), w, scale, c.shift, c.cout, o[c.out_idx] + c.out_off,
                                 c.sb, c.sp, c.sc, ls);
           }
