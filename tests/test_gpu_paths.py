@@ -178,6 +178,29 @@ def test_attention_paths(dtype, b, heads, h, w):
     assert torch.all(out[..., :4] == 7.0) and torch.all(out[..., c + 4:] == 7.0)
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("h,w", [(16, 16), (25, 41)])   # 256 and 1025 keys: eight waves, one and several chunks each
+@pytest.mark.parametrize("lo,hi", [(0, 64), (64, 128), (192, 256), (0, 250)])
+def test_attention_keys_that_score_minus_infinity(dtype, h, w, lo, hi):
+    """Whole chunks of keys whose scores are -inf weigh nothing, whichever wave holds them."""
+    import torch
+    torch.manual_seed(h + lo)
+    qkv = torch.randn(1, h, w, 128, device="cuda").to(tdtype(dtype))
+    qkv[..., 0] = 1.0                                    # q's first channel
+    qkv.view(1, h * w, 128)[:, lo:hi, 32] = -torch.inf   # k's first channel
+    pe_w = torch.zeros(9, 64, device="cuda", dtype=tdtype(dtype))
+    zero = torch.zeros(64, device="cuda")
+    out = torch.zeros(1, h, w, 64, device="cuda", dtype=tdtype(dtype))
+    ctx().psa_attention(vrs.nhwc(qkv), pe_w, zero, zero, vrs.nhwc(out), 1, dtype)
+    q, k, v = qkv.double().reshape(h * w, 128).split((32, 32, 64), 1)
+    keep = torch.ones(h * w, dtype=torch.bool, device="cuda")
+    keep[lo:hi] = False
+    p = (torch.matmul(q, k[keep].t().contiguous()) * 32 ** -0.5).softmax(-1)
+    ref = torch.matmul(p, v[keep].contiguous()).reshape(1, h, w, 64)
+    err = float((out.double() - ref).abs().max() / ref.square().mean().sqrt())
+    assert err < (1e-5 if dtype == vrs.F32 else 4e-2), err   # the bounds of test_attention_paths
+
+
 @pytest.mark.parametrize("h,w,nc,thr,max_det", [
     (64, 96, 5, 0.25, 10),         # 126 anchors: all kept ones sorted
     (96, 160, 80, 0.001, 300),     # 315 anchors (odd)

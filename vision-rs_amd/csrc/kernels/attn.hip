@@ -324,15 +324,17 @@ __device__ __forceinline__ void attn_split_body(const vrs_attn_args& a) {
     cmax = xor_max<32>(cmax);
     // running max in log2 units; p = exp2(s c - m) is one FMA and an exponential,
     // so the only rounding of a score's exponent is that of the difference
-    const float m_new = fmaxf(m_run, cmax * a.scale_log2e);   // finite: the chunk's first key exists
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    const float m_new = fmaxf(m_run, cmax * a.scale_log2e);
+    // (a wave's keys so far may all score -inf: they weigh 0, not exp2(-inf + inf))
+    const float m_ref = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
     m_run = m_new;
     float psum = 0.f;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], a.scale_log2e, -m_new));
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], a.scale_log2e, -m_ref));
         if constexpr (ES == 2) p = bf2f(f2bf(p));   // the sum of exactly what P V consumes
         s[t][r] = p;
         psum += p;
