@@ -156,6 +156,7 @@ def test_depthwise_paths(dtype, n, c, h, w, s):
     (vrs.F32, 1, 1, 23, 23), (vrs.BF16, 1, 1, 23, 23),      # 529 keys: a second round of chunks
     (vrs.BF16, 16, 4, 24, 24),                              # 2304 workgroups of 16 queries: the streamed kernel
     (vrs.BF16, 16, 5, 20, 20),                              # 2000: the resident kernel
+    (vrs.BF16, 13, 1, 50, 50), (vrs.BF16, 11, 1, 50, 50),   # over 2048 keys: 2041 on the streamed kernel, 1727 split
 ])
 def test_attention_paths(dtype, b, heads, h, w):
     import torch

@@ -1115,18 +1115,24 @@ int prep_attn(vrs_ctx* ctx, int heads, int dtype, const vrs_nhwc& qkv, const voi
   char name[48];
   int threads;
   // Split-key kernel (attn.hip): 16 queries per workgroup.  Float32: always
-  // (1.5-4.2x faster than the streamed kernel from 8 to 3200 workgroups, which
-  // stays for images of 2 GiB and more).  bfloat16: while the resident kernel
-  // (up to 512 keys) or the streamed one leaves the chip idle: 20x20 at 4 heads
-  // 800 workgroups 12.6 vs 14.7 us, 1600 20.6 vs 15.3; 37x33 1232 workgroups
-  // 29.7 vs 33.3 us, 30x24 2880 42.8 vs 42.1.  Eight waves share the keys while
-  // that fills at most 8 waves per CU (or there are over 1024 keys), else four:
-  // 20x20 float32 100 workgroups 8.4 vs 8.9 us, 400 14.6 vs 13.6; 9x7 7.0 vs 5.6.
+  // (1.5-4.2x faster than the streamed kernel from 8 to 25600 workgroups of 400
+  // to 25600 keys: 128 x 8 heads at 20x20 457 vs 723 us, 8 x 8 at 80x80 4.53 vs
+  // 7.49 ms; the streamed one stays for images of 2 GiB and more).  bfloat16:
+  // while the resident kernel (up to 512 keys) or the streamed one leaves the
+  // chip idle: 20x20 at 4 heads 800 workgroups 12.6 vs 14.7 us, 1600 20.6 vs
+  // 15.3; over 512 keys up to 8 workgroups per CU (529 keys 2006 25.6 vs 29.8 us,
+  // 1600 keys 2000 53.8 vs 54.7), over 2048, each of them reading all the keys, up
+  // to 7 (2500 keys 1727 69.5 vs 77.0, 2041 78.8 vs 76.7; 3600 keys 1575 95.6 vs
+  // 102, 1800 109 vs 103; 6400 keys 1600 161 vs 169, 2000 184 vs 171), and once a
+  // head's K and V exceed an XCD's 4 MiB L2 up to 6 (11300 keys 1414 240 vs 308,
+  // 25600 keys 1600 618 vs 587).  Eight waves share the keys while that fills at
+  // most 8 waves per CU (or there are over 1024 keys), else four: 20x20 float32 100
+  // workgroups 8.4 vs 8.9 us, 400 14.6 vs 13.6; 9x7 7.0 vs 5.6.
   const int64_t blocks16 = (int64_t)a.B * heads * ((N + 15) / 16);
   const int64_t cus = ctx->num_cu > 0 ? ctx->num_cu : 256;
   const bool image32 = (int64_t)N * qkv.pitch * (int64_t)elt_size(dtype) < (1ll << 31);
   if (image32 && blocks16 < (1ll << 22) &&
-      (dtype == VRS_F32 || blocks16 <= (N <= 512 && a.qkv_bytes > 0 ? 4 : 8) * cus)) {
+      (dtype == VRS_F32 || blocks16 <= (N <= 512 && a.qkv_bytes > 0 ? 4 : N <= 2048 ? 8 : N <= (4 << 20) / 384 ? 7 : 6) * cus)) {
     const int kw = N > 128 && (blocks16 <= cus || (N > 1024 && blocks16 <= 4 * cus)) ? 8 : 4;
     a.q_blocks = (N + 15) / 16;
     threads = kw * 64;
