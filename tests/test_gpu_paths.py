@@ -338,6 +338,22 @@ def test_msda_paths(points, n, q, heads, shapes):
     assert torch.all(out[-8:] == 7.0)
 
 
+def test_msda_of_more_rows_than_a_launch_splits_by_level():
+    """2^23 queries of 8 heads at 8 levels: 2^32 threads with a wave per level."""
+    import oracle
+    import torch
+    from gpu_util import rel_err
+    from test_oracle_golden import msda_inputs
+    q, heads, shapes = 1 << 23, 8, [(2, 3)] * 8
+    value, ref, off, attw = msda_inputs(1, 512, heads, 32, shapes, 1)
+    exp = oracle.msda(value, shapes, ref, off, attw)
+    many = [torch.from_numpy(t).cuda().repeat(1, q // 512, *[1] * (t.ndim - 2)) for t in (ref, off, attw)]
+    out = torch.empty(1, q // 512, 512, heads * 32, device="cuda")
+    ctx().msda(torch.from_numpy(value).cuda(), shapes, *many, out.view(1, q, heads * 32))
+    assert rel_err(out[0, 0].cpu().numpy(), exp[0], 5e-2) < 1e-4   # the bound of test_msda_paths
+    assert torch.equal(out, out[:, :1].expand_as(out))
+
+
 @pytest.mark.parametrize("size,frames", [
     # one canvas tile of the 2x kernel and less; a pixel; a row that no dword fits
     (8, [(16, 16), (1, 1), (3, 1), (5, 16)]),

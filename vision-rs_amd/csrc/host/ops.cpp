@@ -440,18 +440,21 @@ int vrs_msda(vrs_ctx* ctx, const vrs_msda_desc* d, const float* value, const flo
     return fail(VRS_EBADSHAPE, "vrs_msda: value/out must be 16-byte and off 8-byte aligned");
   // 8 lanes per (query, head), each owning 4 of the 32 channels.  Up to 4
   // points: a workgroup per eight (query, head) rows of an image, one wave per
-  // level, an image's values within a buffer load's 32-bit offsets.
-  const int64_t rows = (int64_t)d->q * d->heads;
-  const bool split = d->points <= 4 && rows < (1ll << 31) - 8 && s < (1ll << 31) / (128 * (int64_t)d->heads);
+  // level, an image's values within a buffer load's 32-bit offsets, while its
+  // 64 * levels threads per eight rows stay under the 2^32 of a launch.
+  const int64_t rows = (int64_t)d->q * d->heads, wgs = d->n * ((rows + 7) / 8);
+  const bool split = d->points <= 4 && rows < (1ll << 31) - 8 && s < (1ll << 31) / (128 * (int64_t)d->heads) &&
+                     wgs < (1ll << 32) / (64 * d->levels);
   static const char* const kSplit[] = {"vrs_msda_p1_f32", "vrs_msda_p2_f32", "vrs_msda_p3_f32", "vrs_msda_p4_f32"};
   const char* name = split ? kSplit[d->points - 1] : "vrs_msda_f32";
   hipFunction_t f;
   int rc = get_fn(ctx, name, &f);
   if (rc) return rc;
-  const int64_t blocks = split ? d->n * ((rows + 7) / 8) : (d->n * rows * 8 + 255) / 256;
-  if (blocks >= (1ll << 31)) return fail(VRS_EBADSHAPE, "vrs_msda: grid too large");
+  const int64_t blocks = split ? wgs : (d->n * rows * 8 + 255) / 256;
+  const int threads = split ? 64 * d->levels : 256;
+  if (blocks >= (1ll << 32) / threads) return fail(VRS_EBADSHAPE, "vrs_msda: grid too large");
   std::vector<Launch> ls;
-  ls.push_back(make_launch(name, f, dim3((unsigned)blocks), dim3(split ? 64 * d->levels : 256), 0, a));
+  ls.push_back(make_launch(name, f, dim3((unsigned)blocks), dim3(threads), 0, a));
   return run_all(ls, stream);
 }
 
