@@ -43,6 +43,36 @@ def test_layout_conversions_exact(dtype, n, c, c_pad, h, w, shift):
         assert np.array_equal(back[shift:].cpu().numpy().reshape(n, c - off, h, w), rounder(dtype)(x)[:, off:])
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("n,c,c_pad,h,w,shift", [
+    (1027, 3, 8, 1, 1, 0), (1100, 7, 8, 8, 7, 0),     # 8-channel tiles
+    (1103, 5, 5, 5, 1, 1), (262145, 5, 5, 1, 1, 1),   # rows that no 16-byte chunk fits, an unaligned base; 512 to a tile
+    (700, 130, 136, 1, 1, 0), (603, 64, 68, 3, 5, 0),  # 64-channel tiles, a last one of padding alone
+    (2050, 130, 136, 7, 1, 0), (1050, 9, 9, 3, 7, 1),
+])
+def test_layout_conversions_of_small_maps(dtype, n, c, c_pad, h, w, shift):
+    """Small maps, whole images to a tile: copies, as the larger ones."""
+    test_layout_conversions_exact(dtype, n, c, c_pad, h, w, shift)
+
+
+@pytest.mark.parametrize("n,c,h,w", [(1 << 24, 3, 1, 1), ((1 << 24) + 3, 9, 11, 3)])
+def test_layout_conversions_of_many_maps(n, c, h, w):
+    """2^24 maps and more: calls that take several launches (64-channel tiles of one image)."""
+    import torch
+    part = torch.randn(1 << 12, c, h, w, device="cuda")
+    x = torch.empty(n, c, h, w, device="cuda")
+    for i in range(0, n, 1 << 12):
+        x[i:i + (1 << 12)] = part[:min(1 << 12, n - i)]
+    c_pad = (c + 7) // 8 * 8
+    y = torch.empty(n, h, w, c_pad, dtype=torch.bfloat16, device="cuda")
+    ctx().pack_input(x, vrs.nhwc(y), vrs.BF16)
+    x.zero_()
+    ctx().unpack_output(vrs.nhwc(y, c), vrs.BF16, x)
+    want = part.bfloat16().float()
+    for i in range(0, n, 1 << 12):
+        assert torch.equal(x[i:i + (1 << 12)], want[:min(1 << 12, n - i)])
+
+
 SPLIT_TILES = [pytest.param(vrs.TILE_KW16 | vrs.TILE_SPLIT_1, id="16x4"),
                pytest.param(vrs.TILE_KW16 | vrs.TILE_SPLIT_4, id="16w4"),
                pytest.param(vrs.TILE_KW16 | vrs.TILE_SPLIT_8, id="16w8"),

@@ -971,7 +971,12 @@ int prep_conv_flat(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const vo
 // between the NCHW float32 tensor at `flat` and NHWC rows of `pitch` elements
 // at `rows`.  The 8-channel tile (512 pixels) serves tensors of up to 8
 // channels (images); a 64-channel tile of 64 pixels would leave 7/8 of its
-// lanes without a channel there.
+// lanes without a channel there.  Small maps, where an image fills a small part
+// of a tile, go whole images to a tile (to bfloat16: 3x3 of 64 channels x 16384
+// 32.3 -> 16.1 us, 1x1 of 3 x 65536 65 -> 3.3; but 4x4 of 512 x 4096 37.5 -> 39.2,
+// 5x5 of 512 x 512 11.3 -> 12.3, 11x11 of 8 x 2048 5.1 -> 6.2), unless four
+// workgroups per CU take them one by one (4x4 of 3 x 256 2.5 -> 2.8); fewer to a
+// tile while that leaves the chip less than two workgroups per CU.
 static int prep_layout(vrs_ctx* ctx, const char* op, int dtype, vrs_pack_args& a, int n, int c, int h, int w,
                        int pitch, const void* flat, const void* rows, std::vector<Launch>& out) {
   int rc;
@@ -980,20 +985,30 @@ static int prep_layout(vrs_ctx* ctx, const char* op, int dtype, vrs_pack_args& a
   const int cols = pack ? pitch : c;   // channels written (pack: the zero padding too) or read
   const int ct = cols <= 8 ? 8 : 64, pt = 4096 / ct;
   a.N = n; a.C = c; a.HW = hw; a.c_pad = pitch;
-  const int64_t tp = (hw + pt - 1) / pt;
   a.tiles_c = (cols + ct - 1) / ct;
+  const int64_t cus = ctx->num_cu > 0 ? ctx->num_cu : 256;
+  const bool small = hw <= pt / 2 && hw * std::min(c, ct) < (ct == 8 ? 512 : 1024) && (int64_t)n * a.tiles_c > 4 * cus;
+  a.imgs = small ? (int32_t)(pt / hw) : 1;
+  while (a.imgs > 4 && (int64_t)(n / a.imgs) * a.tiles_c < 2 * cus) a.imgs = (a.imgs + 1) / 2;
+  const int64_t tp = (hw + pt - 1) / pt, groups = ((int64_t)n + a.imgs - 1) / a.imgs;
   const int epc = 16 / elt_size(dtype);
   a.vec_p = hw % 4 == 0 && reinterpret_cast<uintptr_t>(flat) % 16 == 0;
   a.vec_c = pitch % epc == 0 && reinterpret_cast<uintptr_t>(rows) % 16 == 0;
-  const int64_t blocks = (int64_t)n * tp * a.tiles_c;
-  if (blocks >= (1ll << 24)) return fail(VRS_EBADSHAPE, "%s: grid too large", op);   // 2^32 threads
+  const int64_t blocks = groups * tp * a.tiles_c;
+  if (blocks >= (1ll << 31)) return fail(VRS_EBADSHAPE, "%s: grid too large", op);
   a.tiles_p = (int32_t)tp;
   char name[48];
-  snprintf(name, sizeof name, "vrs_%s_nchw_%s_c%d", op, dsuffix(dtype), ct);
+  snprintf(name, sizeof name, "vrs_%s_nchw_%s_%c%d", op, dsuffix(dtype), a.imgs > 1 ? 'i' : 'c', ct);
   hipFunction_t f;
   if ((rc = get_fn(ctx, name, &f))) return rc;
-  out.push_back(make_launch(name, f, dim3((unsigned)blocks), dim3(256), 0, a));
-  out.back().bytes = (double)n * (double)hw * (4.0 * c + (double)cols * elt_size(dtype));
+  const double bytes = (double)n * (double)hw * (4.0 * c + (double)cols * elt_size(dtype));
+  constexpr int64_t kMax = 1ll << 23;   // workgroups of a launch: under 2^32 threads
+  for (int64_t first = 0; first < blocks; first += kMax) {
+    const int64_t count = std::min(kMax, blocks - first);
+    a.first = (uint32_t)first;
+    out.push_back(make_launch(name, f, dim3((unsigned)count), dim3(256), 0, a));
+    out.back().bytes = bytes * (double)count / (double)blocks;
+  }
   return VRS_OK;
 }
 

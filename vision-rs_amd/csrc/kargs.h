@@ -186,7 +186,9 @@ typedef struct {
   void* y;
   int64_t HW;     /* pixels per image */
   int32_t N, C, c_pad;
-  int32_t tiles_p, tiles_c; /* pixel and channel tiles per image */
+  int32_t tiles_p, tiles_c; /* pixel and channel tiles per image (small maps: tiles_c per group of images) */
+  int32_t imgs;   /* small maps: whole images of a tile */
+  uint32_t first; /* first tile of this launch */
   int32_t vec_p;  /* float32 side: 16-byte accesses of 4 pixels (HW % 4 == 0, aligned base) */
   int32_t vec_c;  /* NHWC side: 16-byte accesses of whole channel chunks (aligned base and pitch) */
 } vrs_pack_args;
