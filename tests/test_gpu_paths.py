@@ -179,6 +179,34 @@ def test_depthwise_paths(dtype, n, c, h, w, s):
     assert torch.all(yt[..., c:] == 7.0)
 
 
+@pytest.mark.parametrize("dtype,n,c,h,w,s", [
+    # several images to a tile, the last one of fewer
+    (vrs.F32, 9001, 64, 1, 1, 1), (vrs.F32, 701, 256, 3, 5, 1), (vrs.F32, 211, 136, 9, 7, 1), (vrs.F32, 101, 264, 14, 13, 1),
+    (vrs.F32, 9001, 64, 1, 1, 2), (vrs.F32, 701, 256, 4, 3, 2), (vrs.F32, 401, 136, 7, 9, 2), (vrs.F32, 130, 264, 27, 28, 2),
+    (vrs.BF16, 9001, 64, 1, 1, 1), (vrs.BF16, 701, 256, 5, 3, 1), (vrs.BF16, 211, 136, 8, 9, 1),
+])
+def test_depthwise_small_maps(dtype, n, c, h, w, s):
+    """A period of 37 images against the oracle, the others against it bit for bit."""
+    import oracle
+    import torch
+    from gpu_util import dev, from_nhwc, rel_err, to_nhwc
+    rnd = rounder(dtype)
+    rng = np.random.default_rng([n, c, h, w, s])
+    x = rnd(rng.standard_normal((37, c, h, w), dtype=np.float32))
+    wt = rnd((rng.standard_normal((c, 1, 3, 3)) * 0.4).astype(np.float32))
+    scale = rng.uniform(0.5, 1.5, c).astype(np.float32)
+    shift = rng.normal(0, 0.2, c).astype(np.float32)
+    ref = oracle.affine_act(oracle.conv2d(x, wt, s, 1, c), scale, shift, 1)
+    xt = to_nhwc(x, dtype, c + 8, 8)[torch.arange(n) % 37].contiguous()
+    yt = torch.full((n, ref.shape[2], ref.shape[3], c + 8), 7.0, dtype=tdtype(dtype), device="cuda")
+    ctx().conv2d(vrs.nhwc(xt, c, 8), dev(vrs.pack_conv_weight(wt, c, 1, dtype)), dev(scale), dev(shift),
+                 vrs.nhwc(yt, c, 0), 3, s, c, vrs.ACT_SILU, None, dtype)
+    torch.cuda.synchronize()
+    err = rel_err(from_nhwc(yt[:37], c, 0), ref, 5e-2 if dtype == vrs.F32 else 1e-1)   # bounds of test_depthwise_paths
+    assert err < (1e-4 if dtype == vrs.F32 else 2e-2), err
+    assert torch.equal(yt, yt[:37][torch.arange(n) % 37]) and torch.all(yt[..., c:] == 7.0)
+
+
 @pytest.mark.parametrize("dtype,b,heads,h,w", [
     (vrs.F32, 1, 1, 1, 1), (vrs.BF16, 1, 1, 1, 1),          # one key: three of the four waves have none
     (vrs.F32, 1, 2, 8, 16), (vrs.BF16, 1, 2, 8, 16),        # 128 keys: the last size shared by four waves

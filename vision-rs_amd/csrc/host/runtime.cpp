@@ -817,7 +817,8 @@ static int prep_grouped(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, con
 // of 256 strip parts of four channels) plus, for each further workgroup per CU, its share of loads
 // (t[3]), strips (t[4]) and start (t[5]); microseconds, fitted to 14-17
 // shapes x up to 30 tiles per kernel (rms error 8-10 %; the tile it picks is
-// 1-4 % over the best).
+// 1-4 % over the best).  Maps of up to 12 x 12 may go several images to a
+// workgroup (figures in misc.hip).
 static int64_t dw_tile(int dtype, int stride, int n, int c, int ho, int wo, int num_cu, vrs_dw_args& a) {
   static const double kBf16[6] = {2.25, 0.708, 1.47, 1.86, 0, 0.504}, kF32[6] = {2.26, 1.10, 1.90, 1.76, 0.294, 0.421},
                       kF32s2[6] = {3.01, 1.32, 0.893, 1.14, 0.037, 0.477};
@@ -827,27 +828,30 @@ static int64_t dw_tile(int dtype, int stride, int n, int c, int ho, int wo, int 
   const int64_t blocks = ((int64_t)c * (int64_t)elt_size(dtype) + 63) / 64;
   double best = 1e30;
   int64_t wgs = 0;
-  for (int th0 : {4, 8, 12, 16, 20, 40})
-    for (int tw0 : {10, 16, 20, 32, 40}) {
-      const int th = std::min(th0, ho), tw = std::min(tw0, wo);
-      const int px = ((th - 1) * stride + 3) * ((tw - 1) * stride + 3);
-      if (px * 64 > cap) continue;
-      const int64_t wg = n * blocks * ((ho + th - 1) / th) * ((wo + tw - 1) / tw);
-      const int round = dtype == VRS_BF16 ? 32 : 64;   // strips: a thread takes four channels of 64 bytes
-      const double strips = ((th + 3) / 4 * tw + round - 1) / round;
-      const double us = t[0] + t[1] * ((px + 511) / 512) + t[2] * strips +
-                        std::max(0.0, (double)wg / (num_cu > 0 ? num_cu : 256) - 1.0) *
-                            (t[3] * px / 512 + t[4] * strips + t[5]);
-      if (us < best) {
-        best = us;
-        wgs = wg;
-        a.tile_h = th;
-        a.tile_w = tw;
-        a.cblocks = (int32_t)blocks;
-        a.bands = (ho + th - 1) / th;
-        a.patches = (wo + tw - 1) / tw;
-      }
+  auto offer = [&](int th, int tw, int imgs) {
+    const int px = ((th - 1) * stride + 3) * ((tw - 1) * stride + 3) * imgs;
+    if (px * 64 > cap) return;
+    const int64_t wg = ((int64_t)n + imgs - 1) / imgs * blocks * ((ho + th - 1) / th) * ((wo + tw - 1) / tw);
+    const int round = dtype == VRS_BF16 ? 32 : 64;   // strips: a thread takes four channels of 64 bytes
+    const double strips = ((th + 3) / 4 * tw * imgs + round - 1) / round;
+    const double us = t[0] + t[1] * ((px + 511) / 512) + t[2] * strips +
+                      std::max(0.0, (double)wg / (num_cu > 0 ? num_cu : 256) - 1.0) *
+                          (t[3] * px / 512 + t[4] * strips + t[5]);
+    if (us * (imgs > 1 ? 1.1 : 1.0) < best) {   // (the model's error: not for a small gain)
+      best = us;
+      wgs = wg;
+      a.tile_h = th;
+      a.tile_w = tw;
+      a.imgs = imgs;
+      a.cblocks = (int32_t)blocks;
+      a.bands = (ho + th - 1) / th;
+      a.patches = (wo + tw - 1) / tw;
     }
+  };
+  for (int th0 : {4, 8, 12, 16, 20, 40})
+    for (int tw0 : {10, 16, 20, 32, 40}) offer(std::min(th0, ho), std::min(tw0, wo), 1);
+  if (ho <= 12 && wo <= 12)
+    for (int imgs : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) offer(ho, wo, imgs);
   return wgs;
 }
 
@@ -904,8 +908,9 @@ int prep_conv(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w
     } else {
       const int64_t wgs = dw_tile(cs.dtype, cs.stride, x.n, x.c, y.h, y.w, ctx->num_cu, a);
       if (wgs >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: grid too large");
-      const uint32_t lds = (uint32_t)(((a.tile_h - 1) * cs.stride + 3) * ((a.tile_w - 1) * cs.stride + 3) * 64);
-      snprintf(name, sizeof name, "vrs_dwconv3_t%d_%s", cs.stride, dsuffix(cs.dtype));
+      const uint32_t lds =
+          (uint32_t)(((a.tile_h - 1) * cs.stride + 3) * ((a.tile_w - 1) * cs.stride + 3) * 64 * a.imgs);
+      snprintf(name, sizeof name, "vrs_dwconv3_%c%d_%s", a.imgs > 1 ? 'm' : 't', cs.stride, dsuffix(cs.dtype));
       if ((rc = get_fn(ctx, name, &f))) return rc;
       out.push_back(make_launch(name, f, dim3((unsigned)wgs), dim3(256), lds, a));
     }

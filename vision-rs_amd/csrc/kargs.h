@@ -140,8 +140,9 @@ typedef struct {
    * 8-column patches and row bands per image */
   int32_t x_bytes, cblocks, patches, bands;
   /* LDS-tile kernels: output rows and columns of a tile (cblocks 64-byte
-   * channel blocks, patches x bands tiles per image) */
-  int32_t tile_h, tile_w;
+   * channel blocks, patches x bands tiles per image), or whole images of a
+   * small map */
+  int32_t tile_h, tile_w, imgs;
 } vrs_dw_args;
 
 /* Grouped conv (1 < groups < channels), NHWC, direct form.  x, y, res point

@@ -268,10 +268,15 @@ extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s2_bf16(vrs_dw_arg
 // channels a thread also in bfloat16: with eight, the 72 float weights left two
 // waves per SIMD (11.4 us at 20x20 x 32, 4.9 at 80x80 x 1, 9.8 for 304 channels
 // at 13x11 x 64, now 7.8).
+// MULTI: a tile of several whole images of a small map, else a workgroup has
+// little to do: float32 256 channels at 1x1 x 32768 1573 -> 68 us (walker 594),
+// 3x3 x 3640 200 -> 29 (90), 7x7 x 668 46 -> 26 (30), 10x10 x 327 32 -> 27 (38);
+// stride 2 at 3x3 x 7281 389 -> 39 (a thread per strip 121); bfloat16 3x3 x 3413
+// 59 -> 20.  From 13x13 on the gain is gone (64 MB 23.7 -> 26.4).
 namespace {
 constexpr int DT_R = 4;   // output rows per thread and strip
 
-template <typename T, int S>
+template <typename T, int S, bool MULTI>
 __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
   constexpr int EPC = 4, CB = EPC * (int)sizeof(T), LPP = 64 / CB;   // channels and bytes per thread, threads per pixel
   constexpr int NR = (DT_R - 1) * S + 3;         // input rows of a strip
@@ -282,7 +287,8 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
   const int cb = wg % a.cblocks; wg /= a.cblocks;
   const int tx = wg % a.patches; wg /= a.patches;
   const int ty = wg % a.bands;
-  const int b = wg / a.bands;
+  const int b = MULTI ? wg / a.bands * a.imgs : wg / a.bands;
+  const int imgs = MULTI ? min(a.imgs, a.N - b) : 1;
   const int oy0 = ty * a.tile_h, ox0 = tx * a.tile_w;
   const int ic = (a.tile_w - 1) * S + 3;
   const int rows = min(a.tile_h, a.Ho - oy0), cols = min(a.tile_w, a.Wo - ox0);
@@ -310,23 +316,25 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
   const T* x = reinterpret_cast<const T*>(a.x) + (int64_t)b * a.H * a.W * a.x_pitch + sc0;
   const int iy0 = oy0 * S - 1, ix0 = ox0 * S - 1;
   const float inv_ic = 1.0f / (float)ic;
-  const int npx = ir * ic;
+  const int npx = ir * ic, all = imgs * npx;
+  const float inv_npx = 1.0f / (float)npx;
   constexpr int NB = 8;
-  for (int p0 = tid >> 2; p0 < npx; p0 += 64 * NB) {
+  for (int p0 = tid >> 2; p0 < all; p0 += 64 * NB) {
     u32x4_t v[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       const int p = p0 + i * 64;
-      int cx;
-      const int ry = fdivmod(min(p, npx - 1), ic, inv_ic, cx);
+      int cx, q = min(p, all - 1);
+      const int img = MULTI ? fdivmod(q, npx, inv_npx, q) : 0;
+      const int ry = fdivmod(q, ic, inv_ic, cx);
       const int iy = iy0 + ry, ix = ix0 + cx;
       v[i] = (u32x4_t){0, 0, 0, 0};
-      if (p < npx && sok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W)
-        v[i] = *reinterpret_cast<const u32x4_t*>(x + ((int64_t)iy * a.W + ix) * a.x_pitch);
+      if (p < all && sok && (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W)
+        v[i] = *reinterpret_cast<const u32x4_t*>(x + (((int64_t)img * a.H + iy) * a.W + ix) * a.x_pitch);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i)
-      if (p0 + i * 64 < npx) tile[(p0 + i * 64) * 4 + sch] = v[i];
+      if (p0 + i * 64 < all) tile[(p0 + i * 64) * 4 + sch] = v[i];
   }
   __syncthreads();
   if (!cok) return;
@@ -348,10 +356,11 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
   for (int k = 0; k < 9; ++k) chunk(wq[k], wv[k]);
   T* y = reinterpret_cast<T*>(a.y);
   const int strips = (rows + DT_R - 1) / DT_R, items = strips * cols;
-  const float inv_cols = 1.0f / (float)cols;
-  for (int it = tid / LPP; it < items; it += 256 / LPP) {
-    int ox;
-    const int st = fdivmod(it, cols, inv_cols, ox);
+  const float inv_cols = 1.0f / (float)cols, inv_items = 1.0f / (float)items;
+  for (int it = tid / LPP; it < imgs * items; it += 256 / LPP) {
+    int ox, k = it;
+    const int img = MULTI ? fdivmod(it, items, inv_items, k) : 0;
+    const int st = fdivmod(k, cols, inv_cols, ox);
     float acc[DT_R][EPC];
 #pragma unroll
     for (int r = 0; r < DT_R; ++r)
@@ -362,7 +371,7 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
 #pragma unroll
     for (int rr = 0; rr < NR; ++rr) {
       const int row = min(st * DT_R * S + rr, ir - 1);
-      const part_t* t = reinterpret_cast<const part_t*>(tile) + (row * ic + ox * S) * LPP + ch;
+      const part_t* t = reinterpret_cast<const part_t*>(tile) + (img * npx + row * ic + ox * S) * LPP + ch;
 #pragma unroll
       for (int kx = 0; kx < 3; ++kx) {
         float xv[EPC];
@@ -389,15 +398,18 @@ __device__ __forceinline__ void dwt_body(const vrs_dw_args& a) {
 #pragma unroll
       for (int e = 0; e < CB / 4; ++e)
         o[e] = sizeof(T) == 2 ? pack_bf16x2(v[(2 * e) % EPC], v[(2 * e + 1) % EPC]) : __float_as_uint(v[e]);
-      *reinterpret_cast<part_t*>(y + (((int64_t)b * a.Ho + oy0 + st * DT_R + r) * a.Wo + ox0 + ox) * a.y_pitch + c0) = o;
+      *reinterpret_cast<part_t*>(y + (((int64_t)(b + img) * a.Ho + oy0 + st * DT_R + r) * a.Wo + ox0 + ox) * a.y_pitch + c0) = o;
     }
   }
 }
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(256, 4) void vrs_dwconv3_t1_bf16(vrs_dw_args a) { dwt_body<bf16_t, 1>(a); }
-extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_t1_f32(vrs_dw_args a) { dwt_body<float, 1>(a); }
-extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_t2_f32(vrs_dw_args a) { dwt_body<float, 2>(a); }
+extern "C" __global__ __launch_bounds__(256, 4) void vrs_dwconv3_t1_bf16(vrs_dw_args a) { dwt_body<bf16_t, 1, false>(a); }
+extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_t1_f32(vrs_dw_args a) { dwt_body<float, 1, false>(a); }
+extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_t2_f32(vrs_dw_args a) { dwt_body<float, 2, false>(a); }
+extern "C" __global__ __launch_bounds__(256, 4) void vrs_dwconv3_m1_bf16(vrs_dw_args a) { dwt_body<bf16_t, 1, true>(a); }
+extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_m1_f32(vrs_dw_args a) { dwt_body<float, 1, true>(a); }
+extern "C" __global__ __launch_bounds__(256, 3) void vrs_dwconv3_m2_f32(vrs_dw_args a) { dwt_body<float, 2, true>(a); }
 
 // ---------------------------------------------------------------------------
 // Grouped conv with 1 < groups < channels + folded BN (+ SiLU) (+ residual):
