@@ -157,6 +157,8 @@ def test_split_k_network(tile, dtype):
     (vrs.BF16, 1, 8, 2, 9, 1), (vrs.BF16, 1, 40, 45, 50, 1), (vrs.BF16, 9, 136, 21, 23, 1),
     # row walker (more than 40 MB moved): 10-row bands, and 40-row bands with a 1-row last one
     (vrs.BF16, 12, 320, 33, 90, 1), (vrs.BF16, 16, 264, 41, 75, 1),
+    # float32: the row walker over 512 MB moved
+    (vrs.F32, 41, 264, 79, 83, 1),
 ])
 def test_depthwise_paths(dtype, n, c, h, w, s):
     import oracle

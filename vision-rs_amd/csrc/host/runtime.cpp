@@ -885,24 +885,32 @@ int prep_conv(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w
     a.patches = (x.w + 7) / 8;
     // waves of the row walker on 40-row bands
     const int64_t walk40 = (int64_t)x.n * ((x.h + 39) / 40) * a.cblocks * a.patches;
+    // pixels that an image's 40-row bands of four patches hold
+    const int64_t band_px = (int64_t)((x.h + 39) / 40) * 40 * ((a.patches + 3) / 4) * 32;
+    const bool f32 = cs.dtype == VRS_F32;
+    const bool walker = f32 ? moved > (512ll << 20) && 5ll * x.h * x.w >= 4 * band_px : moved > (40ll << 20);
     const int64_t per_img = (int64_t)((y.h + 3) / 4) * y.w * (x.c / 8);   // 4-row strips of 8 channels
     if (cs.stride == 2 && per_img >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: map too large for one grid row");
     if (cs.dtype == VRS_BF16 && cs.stride == 2) {
       if ((rc = get_fn(ctx, "vrs_dwconv3_s2_bf16", &f))) return rc;
       out.push_back(make_launch("vrs_dwconv3_s2_bf16", f, dim3((unsigned)((per_img + 255) / 256), (unsigned)x.n),
                                 dim3(256), 0, a));
-    } else if (cs.dtype == VRS_BF16 && cs.stride == 1 && xb < (1ll << 31) && moved > (40ll << 20)) {
+    } else if (cs.stride == 1 && xb < (1ll << 31) && walker) {
       // Row-walking kernel: over 40 MB moved it is as fast as the LDS tile or
       // faster (45 MB 17.5 vs 20.4 us, 52 MB 19.9 vs 19.9, 210 MB 52 vs 57;
       // at 26 MB 12.4 vs 11.4).  Bands of 40 output rows on maps of 32 rows or
       // more when that leaves four waves per CU (few band halos and per-wave
       // start-ups; 640 waves 25 us, the same in 10-row bands 18-21 us), else 10.
-      const int rb = x.h >= 32 && walk40 >= 4ll * (ctx->num_cu > 0 ? ctx->num_cu : 256) ? 40 : 10;
+      // float32 (half the rows in flight): over 512 MB, where the maps fill 40-row
+      // bands of four 8-column patches (80x80 839 MB 205 vs 211 us, 1.9 GB 422 vs
+      // 457; 160x160 839 MB 197 vs 205; but 40x40 839 MB 273 vs 205, 20x20 227 vs
+      // 201; 80x80 419 MB 120 vs 111).
+      const int rb = f32 || (x.h >= 32 && walk40 >= 4ll * (ctx->num_cu > 0 ? ctx->num_cu : 256)) ? 40 : 10;
       a.x_bytes = (int32_t)xb;
       a.bands = (x.h + rb - 1) / rb;
       const int64_t wgs = (int64_t)x.n * a.bands * a.cblocks * ((a.patches + 3) / 4);
       if (wgs >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: grid too large");
-      snprintf(name, sizeof name, "vrs_dwconv3_s1w%d_bf16", rb);
+      snprintf(name, sizeof name, "vrs_dwconv3_s1w%d_%s", rb, dsuffix(cs.dtype));
       if ((rc = get_fn(ctx, name, &f))) return rc;
       out.push_back(make_launch(name, f, dim3((unsigned)wgs), dim3(256), 0, a));
     } else {

@@ -100,7 +100,7 @@ __device__ __forceinline__ void dw2_body(const vrs_dw_args& a) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// Stride-1 depthwise 3x3, bfloat16, row walking: large problems.  A wave owns 8 output columns x 64
+// Stride-1 depthwise 3x3, row walking: large problems.  A wave owns 8 output columns x 64
 // channels (lane = channel group g + 8 * column cx) of one band of RB output
 // rows and walks down the band's RB + 2 input rows once: each lane loads its
 // own column (16 bytes per bf16 group), takes the left/right neighbours from
@@ -112,13 +112,13 @@ __device__ __forceinline__ void dw2_body(const vrs_dw_args& a) {
 // flight: two waves per SIMD at ~230 registers), and rows past the band are
 // not fetched.  The four waves of a workgroup take adjacent column patches so
 // their edge columns meet in L1.
-template <int RB>
+template <typename T, int RB>
 __device__ __forceinline__ void dww_body(const vrs_dw_args& a) {
-  using T = bf16_t;
   using E = Elt<T>;
   using G = typename E::group;
   constexpr int NW = (int)sizeof(G) / 4;          // dwords per group
-  constexpr int NP = 6;                           // prefetch ring slots (rows in flight + 1)
+  // prefetch ring slots (rows in flight + 1); float32 rows take twice the registers
+  constexpr int NP = sizeof(T) == 2 ? 6 : 3;
   static_assert((RB + 2) % NP == 0, "rows per band: RB + 2 must be a multiple of the ring");
   // the accumulator slot of band row u (u % 3) is taken from its prefetch
   // slot u % NP at compile time, which needs NP to be a multiple of 3
@@ -245,8 +245,9 @@ __device__ __forceinline__ void dww_body(const vrs_dw_args& a) {
   }
 }
 
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w40_bf16(vrs_dw_args a) { dww_body<40>(a); }
-extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w10_bf16(vrs_dw_args a) { dww_body<10>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w40_bf16(vrs_dw_args a) { dww_body<bf16_t, 40>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w10_bf16(vrs_dw_args a) { dww_body<bf16_t, 10>(a); }
+extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w40_f32(vrs_dw_args a) { dww_body<float, 40>(a); }
 extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s2_bf16(vrs_dw_args a) { dw2_body(a); }
 
 // ---------------------------------------------------------------------------
