@@ -155,8 +155,10 @@ def test_split_k_network(tile, dtype):
     # LDS tile: strips of 4 rows, 64 bytes of channels, tiles of 4..40 x 10..40
     (vrs.F32, 1, 8, 1, 1, 1), (vrs.F32, 1, 24, 45, 50, 1), (vrs.F32, 2, 40, 21, 41, 2), (vrs.F32, 30, 96, 33, 37, 1),
     (vrs.BF16, 1, 8, 2, 9, 1), (vrs.BF16, 1, 40, 45, 50, 1), (vrs.BF16, 9, 136, 21, 23, 1),
-    # row walker (more than 40 MB moved): 10-row bands, and 40-row bands with a 1-row last one
+    # larger ones that do not fill the row walker's bands
     (vrs.BF16, 12, 320, 33, 90, 1), (vrs.BF16, 16, 264, 41, 75, 1),
+    # row walker (over 70 MB moved, bands at least 4/5 filled): 40-row bands, the last of 39 and of 1 row; 10-row bands
+    (vrs.BF16, 16, 264, 79, 90, 1), (vrs.BF16, 9, 136, 281, 90, 1), (vrs.BF16, 61, 264, 29, 63, 1),
     # float32: the row walker over 512 MB moved
     (vrs.F32, 41, 264, 79, 83, 1),
 ])

@@ -883,12 +883,27 @@ int prep_conv(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w
     const int64_t moved = ((int64_t)x.n * x.h * x.w + (int64_t)y.n * y.h * y.w) * x.c * (int64_t)elt_size(cs.dtype);
     a.cblocks = (x.c + 63) / 64;
     a.patches = (x.w + 7) / 8;
-    // waves of the row walker on 40-row bands
-    const int64_t walk40 = (int64_t)x.n * ((x.h + 39) / 40) * a.cblocks * a.patches;
-    // pixels that an image's 40-row bands of four patches hold
-    const int64_t band_px = (int64_t)((x.h + 39) / 40) * 40 * ((a.patches + 3) / 4) * 32;
+    // Row-walking kernel, or the LDS tile?  The walker streams large maps at a
+    // copy's rate where they fill its bands of rb rows x four 8-column patches (by
+    // at least 4/5).  Walker vs tile, bfloat16 256 channels: 80x80 62 MB moved 22.3
+    // vs 21.2 us, 94 MB 34.0 vs 32.0, 125 MB 34.5 vs 40.8, 400 MB 97.6 vs 134;
+    // 160x160 75 MB 22.8 vs 27.4, 300 MB 67.8 vs 87.6; 30x30 129 MB 36.4 vs 46.2.
+    // Where three fifths are filled: 40x40 200 MB 62.2 vs 62.0, 300 MB 93 vs 101;
+    // 80x40 278 MB 91.8 vs 79.2, 400 MB 124 vs 131.  Less: 33x33 128 MB 56.2 vs
+    // 37.6, 400 MB 152 vs 120; 13x13 400 MB 253 vs 115.  float32 (half the rows in
+    // flight, 40-row bands): 80x80 600 MB 165 vs 160, 839 MB 205 vs 211, 1.9 GB 422
+    // vs 457; 160x160 419 MB 109 vs 109, 839 MB 197 vs 205.
+    // Bands of 40 output rows on maps of 32 rows or more when that leaves four
+    // waves per CU (few band halos and per-wave start-ups; 640 waves 25 us, the
+    // same in 10-row bands 18-21 us), else 10.
     const bool f32 = cs.dtype == VRS_F32;
-    const bool walker = f32 ? moved > (512ll << 20) && 5ll * x.h * x.w >= 4 * band_px : moved > (40ll << 20);
+    const int64_t walk40 = (int64_t)x.n * ((x.h + 39) / 40) * a.cblocks * a.patches;   // waves of 40-row bands
+    const int rb = x.h >= 32 && walk40 >= 4ll * (ctx->num_cu > 0 ? ctx->num_cu : 256) ? 40 : 10;
+    a.bands = (x.h + rb - 1) / rb;
+    const int64_t band_px = (int64_t)a.bands * rb * ((a.patches + 3) / 4) * 32, map_px = (int64_t)x.h * x.w;
+    const bool full = 5 * map_px >= 4 * band_px;
+    const bool walker = f32 ? full && rb == 40 && moved > (512ll << 20)
+                            : moved > (full ? 70ll << 20 : 288ll << 20) && 5 * map_px >= 3 * band_px;
     const int64_t per_img = (int64_t)((y.h + 3) / 4) * y.w * (x.c / 8);   // 4-row strips of 8 channels
     if (cs.stride == 2 && per_img >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: map too large for one grid row");
     if (cs.dtype == VRS_BF16 && cs.stride == 2) {
@@ -896,18 +911,7 @@ int prep_conv(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w
       out.push_back(make_launch("vrs_dwconv3_s2_bf16", f, dim3((unsigned)((per_img + 255) / 256), (unsigned)x.n),
                                 dim3(256), 0, a));
     } else if (cs.stride == 1 && xb < (1ll << 31) && walker) {
-      // Row-walking kernel: over 40 MB moved it is as fast as the LDS tile or
-      // faster (45 MB 17.5 vs 20.4 us, 52 MB 19.9 vs 19.9, 210 MB 52 vs 57;
-      // at 26 MB 12.4 vs 11.4).  Bands of 40 output rows on maps of 32 rows or
-      // more when that leaves four waves per CU (few band halos and per-wave
-      // start-ups; 640 waves 25 us, the same in 10-row bands 18-21 us), else 10.
-      // float32 (half the rows in flight): over 512 MB, where the maps fill 40-row
-      // bands of four 8-column patches (80x80 839 MB 205 vs 211 us, 1.9 GB 422 vs
-      // 457; 160x160 839 MB 197 vs 205; but 40x40 839 MB 273 vs 205, 20x20 227 vs
-      // 201; 80x80 419 MB 120 vs 111).
-      const int rb = f32 || (x.h >= 32 && walk40 >= 4ll * (ctx->num_cu > 0 ? ctx->num_cu : 256)) ? 40 : 10;
       a.x_bytes = (int32_t)xb;
-      a.bands = (x.h + rb - 1) / rb;
       const int64_t wgs = (int64_t)x.n * a.bands * a.cblocks * ((a.patches + 3) / 4);
       if (wgs >= (1ll << 24)) return fail(VRS_EBADSHAPE, "dwconv: grid too large");
       snprintf(name, sizeof name, "vrs_dwconv3_s1w%d_%s", rb, dsuffix(cs.dtype));
