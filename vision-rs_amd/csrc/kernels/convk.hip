@@ -154,9 +154,10 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
   }
   u32x4_t va[DEPTH][RL], vb[DEPTH][RL];
   auto load = [&](u32x4_t (&wa)[RL], u32x4_t (&wb)[RL]) {
-    int tap = t_tap, c = t_c;
-    // chunks past K (the last step's tail, steps past the last): zeros
+    // chunks past K (the last step's tail, steps past the last): zeros, at tap 0
+    // (the look-ahead's own tap may be one of no filter)
     uint32_t dead = g < gpr ? 0u : kOOB;
+    int tap = g < gpr ? t_tap : 0, c = t_c;
     if constexpr (!ALIGNED) {
       const int gl = g + ch;
       dead = gl < gpr ? 0u : kOOB;
