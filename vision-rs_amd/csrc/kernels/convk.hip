@@ -189,13 +189,16 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
   constexpr int FB = ES == 1 ? 32 : 16;               // bytes of a row per lane and slice
   const int f_off = (lane % TS) * ROW + (lane / TS) * FB;
   // one step: the staged rows through this wave's own LDS (LDS operations of
-  // one wave are in order: no barrier) into MFMA fragments
+  // one wave are in order: no barrier) into MFMA fragments.  The wave barriers
+  // are for the compiler, which sees only each lane's own addresses: they keep
+  // the stores before the fragment reads and these before the next step's stores.
   auto step = [&](const u32x4_t (&wa)[RL], const u32x4_t (&wb)[RL]) {
 #pragma unroll
     for (int i = 0; i < RL; ++i) {
       *reinterpret_cast<u32x4_t*>(sa + (r0 + 8 * i) * ROW + ch * 16) = wa[i];
       *reinterpret_cast<u32x4_t*>(sb + (r0 + 8 * i) * ROW + ch * 16) = wb[i];
     }
+    __builtin_amdgcn_wave_barrier();
   };
   auto mma = [&]() {
     if constexpr (ES == 1) {
@@ -210,6 +213,7 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
         fa[s] = ld32(sa + f_off + s * NG * FB);
         fb[s] = ld32(sb + f_off + s * NG * FB);
       }
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int s = 0; s < NS; ++s) acc = Unit<T, TS>::mma(fa[s], fb[s], acc);
     } else {
@@ -219,6 +223,7 @@ __device__ __forceinline__ void convk_body(const vrs_convk_args& k) {
         fa[s] = *reinterpret_cast<const u32x4_t*>(sa + f_off + s * NG * 16);
         fb[s] = *reinterpret_cast<const u32x4_t*>(sb + f_off + s * NG * 16);
       }
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int s = 0; s < CPS / NG; ++s) acc = Unit<T, TS>::mma(fa[s], fb[s], acc);
     }
