@@ -377,8 +377,14 @@ static int auto_tile(const ConvSpec& cs, const vrs_conv_args& a, const vrs_nhwc&
   }
   if (f8 && a.kh == 1 && a.stride == 1 && !cs.up && w1_fp8_cin(a.Cin) && !a.res && staged) offer(VRS_TILE_W1_128);
   if (s.dtype == VRS_BF16 && a.kh == 1 && a.stride == 1 && !cs.up && a.Cin % 64 == 0 && !a.res && staged) {
-    if (a.Cin <= 192) offer(VRS_TILE_W1_256);
-    if (a.Cin <= 256 || a.Cin == 384) offer(VRS_TILE_W1_128);
+    // (not with more than one and under three pixel tiles per CU: a stream's
+    // second and third tile cost it more than its later ones, which the model
+    // does not show: 64->256, 12000 pixels 7.8 us, 64x64 tile 5.9; 19000 11.0,
+    // 128x128 8.8; 128->512, 12000 12.1 and 10.1; at 128000 on the W1 tile 29
+    // against 33)
+    auto few = [&](int bm) { return 2 * blocks(bm, 64) > want && 2 * blocks(bm, 64) < 3 * want; };
+    if (a.Cin <= 192 && !few(256)) offer(VRS_TILE_W1_256);
+    if ((a.Cin <= 256 || a.Cin == 384) && !few(128)) offer(VRS_TILE_W1_128);
   }
   return best;
 }
