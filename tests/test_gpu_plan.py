@@ -126,6 +126,26 @@ def test_autotuned_fp8_model_of_small_maps(variant, batch, size, mode):
         assert torch.isfinite(a).all() and torch.equal(a.view(torch.int32), b.view(torch.int32))
 
 
+@pytest.mark.parametrize("batch,size,streams", [(13, (704, 640), 3), (1, (640, 640), 1)])
+def test_default_capture_streams(batch, size, streams):
+    """A small forward is captured as one chain, one of 0.7 ms of work on three streams."""
+    import torch
+    desc = vrs.block(vrs.BLOCK_YOLO26, 3, nc=80, variant="s", one2one=True)
+    m = vrs.Model(ctx(), desc, batch, *size, vrs.BF16, 1e-3, autotune=False)
+    m.load(_params(m))
+    x, outs = torch.rand(batch, 3, *size, device="cuda"), m.alloc_outputs()
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    m.capture(x, outs, stream.cuda_stream)
+    assert m.num_capture_streams() == streams
+    want = [o.clone() for o in m.forward(x)]
+    torch.cuda.synchronize()
+    for _ in range(2):
+        m.replay(stream.cuda_stream)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, want))
+
+
 def test_conv_io_views():
     """conv_io describes each conv: launch order, views inside the model's
     buffers, the stem and the flat Detect outputs."""

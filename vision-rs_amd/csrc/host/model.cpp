@@ -1653,14 +1653,23 @@ int vrs_model_capture(vrs_model* m, const float* x, float* const* outputs, void*
   const int n = (int)m->launches.size();
   // A small forward stays one chain unless the caller asked for streams: its
   // launches are short, and each edge between streams costs more than running
-  // beside the trunk gains (YOLO26n float32 batch 1 573 us on one stream, 651 on
-  // three; YOLO26m bf16 batch 1 690 vs 815, batch 16 2292 vs 2191; YOLO26s bf16
-  // batch 8, about 1 ms, the same).  Small: under 0.75 ms of work at the rates
-  // the kernels reach (600 and 60 TFLOP/s, 4 TB/s).
+  // beside the trunk gains.  Small: under 0.3 ms of work at 600 TFLOP/s in
+  // bfloat16 and fp8, 120 in float32, and 4 TB/s (which the kernels of small
+  // problems are far from: the replays below take three times that and more).
+  // One stream vs three, bfloat16, by work: YOLO26s 320 px batch 13 (0.17 ms) 718
+  // vs 775 us, YOLO26m batch 4 (0.13) 677 vs 786, YOLO26l 640 px batch 1 (0.16)
+  // 939 vs 1019; YOLO26s 640 px batch 6 (0.31) 942 vs 885, YOLO26m batch 4 (0.50)
+  // 1144 vs 1073, batch 16 (2.0) 2292 vs 2169; YOLO26n, whose launches are the
+  // shortest, gains 1-9 % from three at 640 px at any batch.  Float32: YOLO26n
+  // batch 1 566 vs 594, batch 4 925 vs 910, YOLO26s batch 1 794 vs 810, batch 2
+  // 1128 vs 1091.  A Detect head by itself has no trunk to wait for and takes the
+  // streams at any size (of YOLO26m batch 2 169 vs 162, batch 8 289 vs 264; of
+  // YOLO26n batch 32 342 vs 262).
   double work = 0.0;
   for (const Launch& l : m->launches)
-    work += std::max(l.flops / (act_dt(m) == VRS_F32 ? 60e12 : 600e12), l.bytes / 4e12);
-  const int K = !m->streams_set && work < 0.75e-3 ? 1 : std::max(1, std::min(m->streams, 8));
+    work += std::max(l.flops / (act_dt(m) == VRS_F32 ? 120e12 : 600e12), l.bytes / 4e12);
+  const bool small = work < 0.3e-3 && m->desc.kind != VRS_BLOCK_DETECT;
+  const int K = !m->streams_set && small ? 1 : std::max(1, std::min(m->streams, 8));
   auto conflict = [](const LaunchIO& a, const LaunchIO& b) {   // a after b
     auto ov = [](const Access& x, const Access& y) { return x.res == y.res && x.c0 < y.c1 && y.c0 < x.c1; };
     for (const Access& w : a.wr) {
