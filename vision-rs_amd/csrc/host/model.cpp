@@ -1107,23 +1107,33 @@ int autotune_tiles(vrs_model* m) {
     cs.k = c.k; cs.stride = c.s; cs.dtype = dt; cs.act = c.kind == CK_BN_SILU ? VRS_ACT_SILU : VRS_ACT_NONE;
     cs.in_scale = 1.f;  // timing only: values do not matter
     if (pass) e4m3_flags(m, c, cs);   // the storage planned for the forced fp8 model
+    auto prepared = [&](int tile, std::vector<Launch>& ls) {
+      cs.tile = tile;
+      return prep_conv_step(m, c, cs, pass ? c.w8 : c.w, pass ? c.scale8 : c.scale, outs.data(), ls) == VRS_OK;
+    };
     // A small conv's tile is the automatic one when that is a split-K tile,
-    // without a contest: these sum K in another order than the other tiles,
-    // and float32 results must not depend on a timing (all other float32
-    // tiles give the same bits).
-    {
-      std::vector<Launch> ls;
-      if (prep_conv_step(m, c, cs, pass ? c.w8 : c.w, pass ? c.scale8 : c.scale, outs.data(), ls) == VRS_OK &&
-          split_k_tile(ls[0].tile))
-        cand = {ls[0].tile};
+    // without a contest: these sum K in another order than the other tiles, and
+    // a small model's results should not depend on a timing (all other float32
+    // tiles give the same bits).  Else the tiles that this conv takes (its
+    // residual, flat output or fused upsample rule some out) and that are not
+    // predicted far over the best of them.
+    std::vector<Launch> autos;
+    if (prepared(VRS_TILE_AUTO, autos) && split_k_tile(autos[0].tile)) {
+      cand = {autos[0].tile};
+    } else {
+      cand.erase(std::remove_if(cand.begin(), cand.end(),
+                                [&](int t) {
+                                  std::vector<Launch> ls;
+                                  return !prepared(t, ls);
+                                }),
+                 cand.end());
+      if (dt != VRS_FP8) drop_slow_tiles(cand, c.cout, c.cin, dt, c.k, c.s, npix, m->ctx->num_cu);
     }
     float best = 1e30f;
     int best_tile = VRS_TILE_AUTO;
     for (int t : cand) {
-      cs.tile = t;
       std::vector<Launch> ls;
-      if (prep_conv_step(m, c, cs, pass ? c.w8 : c.w, pass ? c.scale8 : c.scale, outs.data(), ls) != VRS_OK)
-        continue;
+      if (!prepared(t, ls)) continue;
       float ms;
       if ((rc = timed(ls, ms))) break;
       // a later candidate must win by 2%: near-ties keep the earlier one, so

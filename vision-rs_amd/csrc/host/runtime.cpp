@@ -433,18 +433,19 @@ std::vector<int> conv_tile_candidates(int cout, int cin, int dtype, int k, int s
       if (t.code == VRS_TILE_128x128 && cin % 64 == 0) c.push_back(t.code | VRS_TILE_PERSIST);
     }
   }
-  // leave out the tiles predicted to take over 1.4 times the best one's time
-  // (nine predictions in ten are within 27 % of the measured time): finalize
-  // times a third to a half of the built tiles
-  if (m > 0) {
-    const ConvShape s{cout, cin, k, dtype, m, m * stride * stride};
-    double best = 1e30;
-    for (int t : c) best = std::min(best, tile_cost(s, t & ~VRS_TILE_PERSIST, 0, num_cu));
-    c.erase(std::remove_if(c.begin(), c.end(),
-                           [&](int t) { return tile_cost(s, t & ~VRS_TILE_PERSIST, 0, num_cu) > 1.4 * best; }),
-            c.end());
-  }
   return c;
+}
+
+// Of the tiles a conv was prepared with, leaves out those predicted to take over
+// 1.4 times the best one's time (nine predictions in ten are within 27 % of the
+// measured time): finalize times a third to a half of the built tiles.
+void drop_slow_tiles(std::vector<int>& c, int cout, int cin, int dtype, int k, int stride, int64_t m, int num_cu) {
+  const ConvShape s{cout, cin, k, dtype, m, m * stride * stride};
+  double best = 1e30;
+  for (int t : c) best = std::min(best, tile_cost(s, t & ~VRS_TILE_PERSIST, 0, num_cu));
+  c.erase(std::remove_if(c.begin(), c.end(),
+                         [&](int t) { return tile_cost(s, t & ~VRS_TILE_PERSIST, 0, num_cu) > 1.4 * best; }),
+          c.end());
 }
 
 // Split-K small-problem kernel (convk.hip) on prep_dense's argument block.

@@ -143,6 +143,7 @@ uint8_t f32_to_e4m3(float v);
 // m: output pixels (0: unknown), num_cu: the device's CUs
 // The split-K tiles (VRS_TILE_KW*) are not among them: see split_k_tile.
 std::vector<int> conv_tile_candidates(int cout, int cin, int dtype, int k, int stride, int w, int64_t m, int num_cu);
+void drop_slow_tiles(std::vector<int>& c, int cout, int cin, int dtype, int k, int stride, int64_t m, int num_cu);
 inline bool split_k_tile(int tile) { return (tile & 0xff) == VRS_TILE_KW32 || (tile & 0xff) == VRS_TILE_KW16; }
 int prep_conv(vrs_ctx* ctx, const ConvSpec& cs, const vrs_nhwc& x, const void* w, const float* scale,
               const float* shift, const vrs_nhwc* res, const vrs_nhwc& y, std::vector<Launch>& out);
