@@ -108,7 +108,7 @@ typedef struct {
  * bit-identical to the tiled fp8 kernels. */
 #define VRS_TILE_W1_256 8
 #define VRS_TILE_W1_128 9
-/* 64x64 tile (bf16, Cin % 32 == 0; 4 waves of 32x32): four times the
+/* 64x64 tile (bf16 and float32, Cin % 32 == 0; 4 waves of 32x32): four times the
  * workgroups of 128x128 for the small maps whose larger tiles leave CUs idle */
 #define VRS_TILE_64x64 10
 /* Model plans only: the conv right after a 64-channel stem (3x3/s2, 64 -> 128,
@@ -162,7 +162,8 @@ typedef struct {
   float in_scale;   /* VRS_FP8: activation quantisation step, a power of two:
                        x8 = rne(clamp(x, +-448*in_scale) / in_scale) */
   /* VRS_FP8 with activations stored as e4m3 (1 byte per channel, views
-   * 16-channel aligned; tiles 128x128, 256x128, 128x256, 64x256, 256x256):
+   * 16-channel aligned; tiles 128x128, 256x128, 128x256, 64x256, 256x256 and,
+   * with x_e4m3, the split-K ones):
    * x_e4m3 -- x (and a fused-upsample source) already holds e4m3 on step
    * in_scale; y_e4m3 -- y is written as rne(clamp(y, +-448*out_step) /
    * out_step) of its bfloat16 value; res_e4m3 -- res holds e4m3 on step
@@ -231,7 +232,9 @@ int vrs_conv_stem(vrs_ctx* ctx, const vrs_conv_desc* d, const float* x_nchw, int
  * network's largest activation) is never written to memory.
  *   y = silu(scale1 * conv3x3s2(s, w1) + shift1),
  *   s = bf16(silu(scale0 * conv3x3s2(x, w0) + shift0))
- * with the same results as the two calls.  w0 from vrs_pack_stem_weight
+ * with the same results as the two calls, the second on any tile but the
+ * split-K ones (which VRS_TILE_AUTO may take for small images, and which sum
+ * in another order).  w0 from vrs_pack_stem_weight
  * (Cout 64), w1 from vrs_pack_conv_weight ([128][3][3][64]); y: 128 channels,
  * image width a multiple of 4. */
 int vrs_conv_stem_pair(vrs_ctx* ctx, const vrs_conv_desc* d0, const vrs_conv_desc* d1, const float* x_nchw,
@@ -428,8 +431,11 @@ int vrs_model_create(vrs_ctx* ctx, const vrs_block_desc* d, int32_t batch, int32
                      int32_t dtype, float bn_eps, vrs_model** out);
 /* Per-layer tile autotuning at finalize (replaces TritonLowering's
  * shape-adaptive tile choice, examples/yolo26.rs:3027).  mode 1 (default):
- * every dense conv is timed with each applicable VRS_TILE_* on the model's own
- * buffers and the fastest is kept; in a VRS_FP8 model each eligible conv also
+ * every dense conv is timed with the VRS_TILE_* that it takes on the model's own
+ * buffers and the fastest is kept, but for bf16 and float32 tiles predicted to
+ * take over 1.4 times the best one's time, and for convs whose automatic tile is
+ * a split-K one: these take it untimed, so that a small model's results do not
+ * depend on a timing.  In a VRS_FP8 model each eligible conv also
  * keeps bf16 when its best bf16 tile is faster.  mode 2 (VRS_FP8 models):
  * only fp8 tiles are timed and every eligible conv runs on fp8, except the
  * conv after a 64-channel stem when the stem pair (VRS_TILE_STEM_PAIR, a bf16

@@ -1146,7 +1146,8 @@ LB_SIZES = [(1280, 720), (640, 640), (517, 333), (333, 517), (1000, 37), (5, 3),
 def test_letterbox():
     """Letterbox preprocessing of 24 images of mixed sizes, bit-exact against
     the oracle's two-pass restatement of the Triangle resize, through every
-    kernel: enlargements and shrinks up to 2x (staged, 64-wide tiles), up to 4x
+    kernel but the one for calls without a shrink (test_letterbox_paths):
+    enlargements and shrinks up to 2x (staged, 64-wide tiles), up to 4x
     (1920 and exactly 4x at 2560 wide), up to 8x (2600, 4000, exactly 8x at
     5120 wide: 32-wide tiles) and beyond (6000 wide: direct kernel); the
     identity, 1x1, thin strips, saturated regions, odd byte offsets."""
@@ -1190,9 +1191,9 @@ def test_letterbox_rejections():
 
 
 @pytest.mark.parametrize("cfg", [
-    (2, 30, 4, [(16, 16), (8, 8), (4, 4), (2, 2)], 4),   # level-split kernel (one wave per level)
-    (1, 6, 16, [(9, 9), (5, 5), (3, 3), (2, 2)], 4),     # unrolled 4x4 kernel (> 8 heads)
-    (1, 7, 8, [(13, 11), (7, 6)], 3),                    # generic kernel
+    (2, 30, 4, [(16, 16), (8, 8), (4, 4), (2, 2)], 4),   # a wave per level, two queries to a workgroup
+    (1, 6, 16, [(9, 9), (5, 5), (3, 3), (2, 2)], 4),     # a query's rows over two workgroups
+    (1, 7, 8, [(13, 11), (7, 6)], 3),                    # two levels, three points
     (1, 5, 8, [(80, 80), (40, 40), (20, 20), (10, 10)], 4),  # BASELINE config 4 level shapes
 ])
 def test_msda(cfg):

@@ -1114,7 +1114,10 @@ int autotune_tiles(vrs_model* m) {
     // A small conv's tile is the automatic one when that is a split-K tile,
     // without a contest: these sum K in another order than the other tiles, and
     // a small model's results should not depend on a timing (all other float32
-    // tiles give the same bits).  Else the tiles that this conv takes (its
+    // tiles give the same bits).  In bfloat16 six of 197 such layers of the n, s
+    // and m networks are over 8 % slower than their best other tile (3x3/s2
+    // 512->512 at 80x80 x 1 31 us, 64x64 tile 27), yet timing them against the
+    // others made no network faster.  Else the tiles that this conv takes (its
     // residual, flat output or fused upsample rule some out) and that are not
     // predicted far over the best of them.
     std::vector<Launch> autos;

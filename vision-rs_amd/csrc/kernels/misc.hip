@@ -251,8 +251,8 @@ extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s1w40_f32(vrs_dw_a
 extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s2_bf16(vrs_dw_args a) { dw2_body(a); }
 
 // ---------------------------------------------------------------------------
-// Depthwise 3x3 through an LDS tile: float32, and bfloat16 stride 1 where the
-// row walker's waves do not fill the chip.  A walker wave takes 12 or 42 rows
+// Depthwise 3x3 through an LDS tile: float32, and bfloat16 stride 1, but for the
+// large maps that fill the row walker's bands.  A walker wave takes 12 or 42 rows
 // one after the other, so a small problem took 8 or 23 us whatever its size
 // (float32, with fewer rows in flight, 12 or 39 us).  Here a workgroup takes 64
 // bytes of channels (4 chunks of 16 bytes) of a tile_h x tile_w output tile:
@@ -265,7 +265,7 @@ extern "C" __global__ __launch_bounds__(256) void vrs_dwconv3_s2_bf16(vrs_dw_arg
 // 117 -> 109 us; stride 2 (one thread per output strip before) 512 at 40x40 x 1
 // 8.5 -> 5.4 us, 256 at 80x80 x 32 77 -> 58 us; bfloat16 64 at 80x80 x 1 22.5 ->
 // 4.4 us, 256 at 80x80 x 4 24.3 -> 11.1 us, 512 at 20x20 x 32 12.5 -> 10.8 us
-// (a copy of it 7.5), 256 at 80x80 x 32 52 -> 57 us (walker kept).  Four
+// (a copy of it 7.5), 256 at 80x80 x 64 98 -> 134 us (walker kept).  Four
 // channels a thread also in bfloat16: with eight, the 72 float weights left two
 // waves per SIMD (11.4 us at 20x20 x 32, 4.9 at 80x80 x 1, 9.8 for 304 channels
 // at 13x11 x 64, now 7.8).

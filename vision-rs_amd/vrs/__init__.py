@@ -36,7 +36,7 @@ TILE_K128 = 0x400   # fp8: 128-deep K steps (256x256 with e4m3 input, Cin % 128 
 TILE_H3 = 7   # halo-tiled 3x3 stride-1 kernel (bf16)
 TILE_W1_256 = 8   # weight-stationary 1x1 kernels (bf16): 256- or 128-channel weight slice in LDS
 TILE_W1_128 = 9
-TILE_64x64 = 10   # bf16: small maps (four times the workgroups of 128x128)
+TILE_64x64 = 10   # bf16, float32: small maps (four times the workgroups of 128x128)
 TILE_KW32 = 14   # split-K kernels for small problems: one 32x32 or 16x16 tile per workgroup
 TILE_KW16 = 15
 TILE_SPLIT_1, TILE_SPLIT_4, TILE_SPLIT_8 = 0x1000, 0x2000, 0x3000   # OR: waves sharing K
